@@ -123,11 +123,19 @@ __device__ __forceinline__ uint32_t pk_bf16(float a, float b)
 }
 
 // Two exponentials as hi and lo bf16 halves, hi = bf16(e), lo = bf16(e - hi),
-// each pair packed (e0 low, e1 high).
+// each pair packed (e0 low, e1 high). e - hi is one v_dot2_f32_bf16 of the
+// packed pair with (-1, 0) or (0, -1), where unpacking and subtracting take
+// two instructions per value; the difference is exact either way.
 __device__ __forceinline__ void split2(float e0, float e1, uint32_t &hi, uint32_t &lo)
 {
     hi = pk_bf16(e0, e1);
-    lo = pk_bf16(e0 - __uint_as_float(hi << 16), e1 - __uint_as_float(hi & 0xFFFF0000u));
+    const bf16x2 h = __builtin_bit_cast(bf16x2, hi);
+    // (constants kept in scalar registers: as inline constants of the packed
+    // operand they would not name the half meant)
+    uint32_t c0 = 0x0000BF80u, c1 = 0xBF800000u;
+    asm("" : "+s"(c0), "+s"(c1));
+    lo = pk_bf16(__builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(bf16x2, c0), e0, false),
+                 __builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(bf16x2, c1), e1, false));
 }
 
 // Eight exponentials as hi and lo bf16 halves, packed in k order.
@@ -1898,45 +1906,62 @@ __global__ __launch_bounds__(512) void decode_combine(DecodeArgs a)
 // tiles from LDS. Tiles are double-buffered: the global loads of tile t+1 are
 // in flight while tile t is computed. Tiles below the diagonal of all of a
 // wave's rows skip the causal mask.
-// POW2 (the scale is a positive power of two): fl(fl(dot * scale) - M) equals
-// fl(dot - Mraw) * scale exactly, Mraw being the maximum of the unscaled
-// dot products, and the scale folds exactly into the exponential's clamp
-// (-87.33654 / scale) and multiplier (log2(e) * scale). Otherwise every score
-// is scaled first, as in the reference.
+// The kernels keep the unscaled dot products: q takes the scale's sign as it
+// is loaded (q_sign; |scale| below), so the row maximum of fl(dot * |scale|)
+// is fl(Mraw * |scale|), the rounding being monotonic. An exponential then
+// takes one fused step from the dot product to the exponent, t = dot * c + b
+// with c = |scale| log2(e) and b = 1/2 - Mraw c.
 // ---------------------------------------------------------------------------
-struct ExpArgs {
-    float m;        // POW2: Mraw; otherwise the scaled maximum M
-    float scale;    // otherwise: the scale
-    float clamp;    // POW2: -87.33654 / scale; otherwise -87.33654
-    float mul;      // POW2: 1.442695 * scale; otherwise 1.442695
-};
-
-template <bool POW2>
-__device__ __forceinline__ float exp_score(float acc, const ExpArgs &x)
+__device__ __forceinline__ uint32_t q_sign(const PrefillArgs &a) { return a.scale < 0.0f ? 0x80008000u : 0u; }
+__device__ __forceinline__ u32x4 q_chunk(u32x4 v, bool valid, uint32_t sign)
 {
-    const float d = POW2 ? acc - x.m : acc * x.scale - x.m;
-    const float t1 = __builtin_fmaxf(d, x.clamp) * x.mul;
-    const float t2 = __builtin_rintf(t1);
-    const float f = t1 - t2;
-    float p = __builtin_fmaf(f, 0.00967248f, 0.05550411f);
-    p = __builtin_fmaf(f, p, 0.2402265f);
-    p = __builtin_fmaf(f, p, 0.6931472f);
-    p = __builtin_fmaf(f, p, 1.0f);
-    return __builtin_ldexpf(p, static_cast<int>(t2));
+    return valid ? v ^ sign : u32x4{0, 0, 0, 0};
 }
 
-// The sink joins a causal row's maximum m (under POW2 the maximum of the
-// unscaled dot products, as the kernels keep it): the scaled maximum becomes
-// the larger of M and the sink (vmaxss, decode.rs:239-290), returned in ms;
-// the result is the maximum the exponentials take, ms / scale under POW2
-// (exact for a power of two; a quotient past the f32 range is infinite, and
-// every exponential then clamps as the reference's does).
-template <bool POW2>
-__device__ __forceinline__ float sink_max(float m, const PrefillArgs &a, float &ms)
+// One row's exponential: see exp_score.
+struct RowExp {
+    float c, b;
+    // m: the row's maximum dot product; with the sink, ms receives the scaled
+    // maximum, the larger of the scores' and the sink (vmaxss,
+    // decode.rs:239-290). Where the exponent of the maximum itself would leave
+    // the f32 range, two scores that differ at all differ by far more than the
+    // exponential's clamp, and a smaller c tells them apart as well.
+    __device__ __forceinline__ RowExp(const PrefillArgs &a, float m, bool sink, float &ms)
+    {
+        const float s = __builtin_fabsf(a.scale);
+        c = s * 1.442695f;
+        const float sm = m * s;
+        const bool over = sink && !(sm > a.sink);
+        ms = over ? a.sink : sm;
+        float t = over ? a.sink * 1.442695f : m * c;
+        if (__builtin_fabsf(t) > 1e38f) {
+            c *= 0x1p-24f;
+            t = over ? a.sink * (1.442695f * 0x1p-24f) : m * c;
+        }
+        b = 0.5f - t;
+    }
+};
+
+// P(x - M) of the score x whose dot product is acc: t = (x - M) log2(e) + 1/2
+// in one rounding, clamped as the emitted exponential clamps (a NaN too), k =
+// floor(t), and the emitted polynomial about t - k - 1/2, its argument moved
+// by 1/2 into the coefficients: P(x) 2^k = Q(t - k) 2^k. Nine instructions
+// where subtract, clamp, scale, round, subtract, convert, polynomial and
+// ldexp take eleven (and one more for a scale that is no power of two): the
+// causal passes are VALU-bound up to D = 128. Against 64-bit exponentials over
+// |score - M| up to 30, relative rms 1.42e-5 and largest 6.1e-5, both the
+// polynomial's own and the same either way.
+__device__ __forceinline__ float exp_score(float acc, const RowExp &x)
 {
-    const float s = POW2 ? m * a.scale : m;
-    ms = s > a.sink ? s : a.sink;
-    return POW2 ? ms / a.scale : ms;
+    const float t = __builtin_fmaxf(__builtin_fmaf(acc, x.c, x.b), -125.49977f);
+    int k;
+    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(k) : "v"(t));
+    const float f = __builtin_amdgcn_fractf(t);
+    float p = __builtin_fmaf(f, 0.00967248f, 0.03615915f);
+    p = __builtin_fmaf(f, p, 0.17147906f);
+    p = __builtin_fmaf(f, p, 0.4897125f);
+    p = __builtin_fmaf(f, p, 0.70714957f);
+    return __builtin_ldexpf(p, k);
 }
 
 // A row's normalisation: the division by its sum, or (the sink) the
@@ -1973,114 +1998,45 @@ __device__ __forceinline__ void store_rows(const f32x16 *o, uint16_t *op, const 
         }
 }
 
-template <int D, int HPW, bool POW2, int NW = 8, bool SINK = false>
-__global__ __launch_bounds__(64 * NW, 1) void prefill_attn(PrefillArgs a)
+// The tiles [tb, te) of one row block's key range: scores, exponentials at the
+// exact maximum and P.V with P = hi + lo, added to o and lsum. K rows past the
+// cache read row 0 and are never visible, V rows past it are zeroed. Every
+// wave of the workgroup walks the same tiles; a wave's tiles from nfull on
+// take the masked path.
+template <int D, int NW>
+__device__ __forceinline__ void pv_walk(const PrefillArgs &a, const uint16_t *kg, const uint16_t *vg,
+                                        uint16_t (*kb)[kKeyTile * Pad<D>::K], uint16_t (*vb)[kKeyTile * Pad<D>::V],
+                                        const u32x4 (&qb)[D / 16], const RowExp &ex, uint64_t lim, int nfull, int tb,
+                                        int te, int tid, f32x16 (&o)[D / 32], float &lsum)
 {
-    constexpr int RB = NW / HPW, THREADS = 64 * NW;
+    constexpr int THREADS = 64 * NW;
     constexpr int SK = Pad<D>::K, SV = Pad<D>::V;
-    __shared__ __attribute__((aligned(16))) uint16_t kb[2][kKeyTile * SK];
-    __shared__ __attribute__((aligned(16))) uint16_t vb[2][kKeyTile * SV];
-    const int tid = threadIdx.x;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, col = l & 31, grp = l >> 5;
-    const int head = blockIdx.y * HPW + (wave % HPW);
-    const int kvh = head / a.gqa;
-    const uint64_t rgroup = gridDim.x - 1 - blockIdx.x;       // heaviest rows first
-    const uint64_t wg_r0 = rgroup * (32 * RB);
-    const uint64_t w_r0 = wg_r0 + 32 * (wave / HPW);
-    const uint64_t row = w_r0 + col;
-    const bool rowv = row < a.rows;
-    const bool wact = w_r0 < a.rows;
-    const uint64_t wg_rend = wg_r0 + 32 * RB < a.rows ? wg_r0 + 32 * RB : a.rows;
-    const int ntiles = static_cast<int>((a.past + wg_rend + kKeyTile - 1) / kKeyTile);
-    const int nfull = wact ? static_cast<int>((a.past + w_r0 + 1) / kKeyTile) : 0;  // no mask needed
-    const uint64_t lim = a.past + row;                         // last visible key of this row
-
-    const uint16_t *kg = a.k + static_cast<uint64_t>(kvh) * a.kv_stride;
-    const uint16_t *vg = a.v + static_cast<uint64_t>(kvh) * a.kv_stride;
-    u32x4 kr[Tile<D, THREADS>::kPer], vr[Tile<D, THREADS>::kPer];
-    u32x4 qb[D / 16];
-    const uint16_t *qp = a.q + (rowv ? row : 0) * a.q_row + static_cast<uint64_t>(head) * a.q_head;
-#pragma unroll
-    for (int s = 0; s < D / 16; s++) {
-        const u32x4 v = load16(qp + 16 * s + 8 * grp);
-        qb[s] = rowv ? v : u32x4{0, 0, 0, 0};
-    }
-    tile_gload<D, THREADS, false>(kg, 0, a.n, tid, kr);
+    const int l = tid & 63, col = l & 31, grp = l >> 5;
     const int arow = swap23(col) * SK + 8 * grp;
-    // One accumulation chain: a second one would not fit the 256 registers
-    // of two waves per SIMD; the other wave on the SIMD fills the gaps.
-    auto qk = [&](const uint16_t *kt) {
+    u32x4 kr[Tile<D, THREADS>::kPer], vr[Tile<D, THREADS>::kPer];
+    tile_gload<D, THREADS, false>(kg, static_cast<uint64_t>(tb) * kKeyTile, a.n, tid, kr);
+    tile_gload<D, THREADS, false>(vg, static_cast<uint64_t>(tb) * kKeyTile, a.n, tid, vr);
+    // The next K tile is loaded first, the next V tile after the first half's
+    // exponentials, so that their staging registers are not live at the peak;
+    // the loads are not branched around, the masked and unmasked halves of a
+    // tile are instantiated apart, and the products run at raised priority.
+    tile_lstore_padded<D, THREADS>(kb[0], SK, tid, kr);
+    tile_mask<D, THREADS>(static_cast<uint64_t>(tb) * kKeyTile, a.n, tid, vr);
+    tile_lstore_padded<D, THREADS>(vb[0], SV, tid, vr);
+    __syncthreads();
+    for (int t = tb; t < te; t++) {
+        const uint64_t t0 = static_cast<uint64_t>(t) * kKeyTile;
+        const int b = (t - tb) & 1;
+        tile_gload<D, THREADS, false>(kg, t0 + kKeyTile, a.n, tid, kr);  // past the cache: row 0, unused
+        __builtin_amdgcn_sched_barrier(0);
         f32x16 acc = {};
 #pragma unroll
         for (int s = 0; s < D / 16; s += 2) {
             // two K operands requested before their MFMAs
-            const u32x4 k0 = load16(kt + arow + 16 * s), k1 = load16(kt + arow + 16 * (s + 1));
+            const u32x4 k0 = load16(kb[b] + arow + 16 * s), k1 = load16(kb[b] + arow + 16 * (s + 1));
             acc = mfma(k0, qb[s], acc);
             acc = mfma(k1, qb[s + 1], acc);
         }
-        return acc;
-    };
-
-    // Every wave computes every tile of the workgroup's key range: tiles past
-    // a wave's last visible key take the masked path and contribute nothing.
-    // With no wave-dependent branches around them, the loads of the next
-    // tiles stay in flight across the compute.
-
-    // pass 1: exact row maxima (of the unscaled dot products when POW2).
-    // Out-of-range keys of the last tile read row 0 and are never visible.
-    tile_lstore_padded<D, THREADS>(kb[0], SK, tid, kr);
-    __syncthreads();
-    float m = kNegInf;
-    for (int t = 0; t < ntiles; t++) {
-        const uint64_t t0 = static_cast<uint64_t>(t) * kKeyTile;
-        const bool last = t + 1 == ntiles;
-        tile_gload<D, THREADS, false>(kg, last ? 0 : t0 + kKeyTile, a.n, tid, kr);   // after the last: pass 2's first tile
-        if (last) tile_gload<D, THREADS, false>(vg, 0, a.n, tid, vr);
-        __builtin_amdgcn_sched_barrier(0);
-        const f32x16 acc = qk(kb[t & 1]);
-        if (t < nfull) {
-#pragma unroll
-            for (int r = 0; r < 16; r++) m = __builtin_fmaxf(m, POW2 ? acc[r] : acc[r] * a.scale);
-        } else {
-            // keys t0 + k with k <= vis are visible to this row
-            const int vis = static_cast<int>(static_cast<int64_t>(lim) - static_cast<int64_t>(t0));
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const float s = POW2 ? acc[r] : acc[r] * a.scale;
-                if (key_of(r, grp) <= vis) m = __builtin_fmaxf(m, s);
-            }
-        }
-        if (!last) tile_lstore_padded<D, THREADS>(kb[(t + 1) & 1], SK, tid, kr);
-        __syncthreads();
-    }
-    m = __builtin_fmaxf(m, __shfl_xor(m, 32));
-    float ms = 0.0f;                                            // the scaled maximum, with the sink
-    if constexpr (SINK) m = sink_max<POW2>(m, a, ms);
-    ExpArgs ex;
-    ex.m = m;
-    ex.scale = a.scale;
-    ex.clamp = POW2 ? -87.33654f / a.scale : -87.33654f;
-    ex.mul = POW2 ? 1.442695f * a.scale : 1.442695f;
-
-    // pass 2: exponentials at the exact maximum, P.V with P = hi + lo. The
-    // next K tile is loaded first, the next V tile after the first half's
-    // softmax, so that their staging registers are not live at the peak.
-    tile_lstore_padded<D, THREADS>(kb[0], SK, tid, kr);
-    tile_mask<D, THREADS>(0, a.n, tid, vr);
-    tile_lstore_padded<D, THREADS>(vb[0], SV, tid, vr);
-    __syncthreads();
-    f32x16 o[D / 32];
-#pragma unroll
-    for (int dt = 0; dt < D / 32; dt++) o[dt] = f32x16{};
-    // the sink's exponential starts the row's sum (in one of its two lanes),
-    // so that nothing of it stays live across the tiles
-    float lsum = SINK && grp == 0 ? exp_poly(a.sink - ms) : 0.0f;
-    for (int t = 0; t < ntiles; t++) {
-        const uint64_t t0 = static_cast<uint64_t>(t) * kKeyTile;
-        const int b = t & 1;
-        tile_gload<D, THREADS, false>(kg, t0 + kKeyTile, a.n, tid, kr);  // past the end: row 0, unused
-        __builtin_amdgcn_sched_barrier(0);
-        const f32x16 acc = qk(kb[b]);
         const bool full = t < nfull;
         const int vis = static_cast<int>(static_cast<int64_t>(lim) - static_cast<int64_t>(t0));
         // exponentials of one half of the tile's keys as hi and lo operands
@@ -2089,7 +2045,7 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_attn(PrefillArgs a)
             float ev[8];
 #pragma unroll
             for (int r = 0; r < 8; r++) {
-                const float e = exp_score<POW2>(acc[8 * h + r], ex);
+                const float e = exp_score(acc[8 * h + r], ex);
                 ev[r] = !MASKED || key_of(8 * h + r, grp) <= vis ? e : 0.0f;
                 lsum += ev[r];
             }
@@ -2114,13 +2070,104 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_attn(PrefillArgs a)
         if (full) half(1, std::false_type{}, hi, lo);
         else half(1, std::true_type{}, hi, lo);
         pv(1, hi, lo);
-        if (t + 1 < ntiles) {
+        if (t + 1 < te) {
             tile_lstore_padded<D, THREADS>(kb[b ^ 1], SK, tid, kr);
             tile_mask<D, THREADS>(t0 + kKeyTile, a.n, tid, vr);
             tile_lstore_padded<D, THREADS>(vb[b ^ 1], SV, tid, vr);
         }
         __syncthreads();
     }
+}
+
+template <int D, int HPW, int NW = 8, bool SINK = false>
+__global__ __launch_bounds__(64 * NW, 1) void prefill_attn(PrefillArgs a)
+{
+    constexpr int RB = NW / HPW, THREADS = 64 * NW;
+    constexpr int SK = Pad<D>::K, SV = Pad<D>::V;
+    __shared__ __attribute__((aligned(16))) uint16_t kb[2][kKeyTile * SK];
+    __shared__ __attribute__((aligned(16))) uint16_t vb[2][kKeyTile * SV];
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, col = l & 31, grp = l >> 5;
+    const int head = blockIdx.y * HPW + (wave % HPW);
+    const int kvh = head / a.gqa;
+    const uint64_t rgroup = gridDim.x - 1 - blockIdx.x;       // heaviest rows first
+    const uint64_t wg_r0 = rgroup * (32 * RB);
+    const uint64_t w_r0 = wg_r0 + 32 * (wave / HPW);
+    const uint64_t row = w_r0 + col;
+    const bool rowv = row < a.rows;
+    const bool wact = w_r0 < a.rows;
+    const uint64_t wg_rend = wg_r0 + 32 * RB < a.rows ? wg_r0 + 32 * RB : a.rows;
+    const int ntiles = static_cast<int>((a.past + wg_rend + kKeyTile - 1) / kKeyTile);
+    const int nfull = wact ? static_cast<int>((a.past + w_r0 + 1) / kKeyTile) : 0;  // no mask needed
+    const uint64_t lim = a.past + row;                         // last visible key of this row
+
+    const uint16_t *kg = a.k + static_cast<uint64_t>(kvh) * a.kv_stride;
+    const uint16_t *vg = a.v + static_cast<uint64_t>(kvh) * a.kv_stride;
+    u32x4 kr[Tile<D, THREADS>::kPer];
+    u32x4 qb[D / 16];
+    const uint16_t *qp = a.q + (rowv ? row : 0) * a.q_row + static_cast<uint64_t>(head) * a.q_head;
+#pragma unroll
+    for (int s = 0; s < D / 16; s++) {
+        const u32x4 v = load16(qp + 16 * s + 8 * grp);
+        qb[s] = q_chunk(v, rowv, q_sign(a));
+    }
+    tile_gload<D, THREADS, false>(kg, 0, a.n, tid, kr);
+    const int arow = swap23(col) * SK + 8 * grp;
+    // One accumulation chain: a second one would not fit the 256 registers
+    // of two waves per SIMD; the other wave on the SIMD fills the gaps.
+    auto qk = [&](const uint16_t *kt) {
+        f32x16 acc = {};
+#pragma unroll
+        for (int s = 0; s < D / 16; s += 2) {
+            // two K operands requested before their MFMAs
+            const u32x4 k0 = load16(kt + arow + 16 * s), k1 = load16(kt + arow + 16 * (s + 1));
+            acc = mfma(k0, qb[s], acc);
+            acc = mfma(k1, qb[s + 1], acc);
+        }
+        return acc;
+    };
+
+    // Every wave computes every tile of the workgroup's key range: tiles past
+    // a wave's last visible key take the masked path and contribute nothing.
+    // With no wave-dependent branches around them, the loads of the next
+    // tiles stay in flight across the compute.
+
+    // pass 1: exact row maxima of the unscaled dot products.
+    // Out-of-range keys of the last tile read row 0 and are never visible.
+    tile_lstore_padded<D, THREADS>(kb[0], SK, tid, kr);
+    __syncthreads();
+    float m = kNegInf;
+    for (int t = 0; t < ntiles; t++) {
+        const uint64_t t0 = static_cast<uint64_t>(t) * kKeyTile;
+        const bool last = t + 1 == ntiles;
+        tile_gload<D, THREADS, false>(kg, t0 + kKeyTile, a.n, tid, kr);   // past the cache: row 0, unused
+        __builtin_amdgcn_sched_barrier(0);
+        const f32x16 acc = qk(kb[t & 1]);
+        if (t < nfull) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) m = __builtin_fmaxf(m, acc[r]);
+        } else {
+            // keys t0 + k with k <= vis are visible to this row
+            const int vis = static_cast<int>(static_cast<int64_t>(lim) - static_cast<int64_t>(t0));
+#pragma unroll
+            for (int r = 0; r < 16; r++) 
+                if (key_of(r, grp) <= vis) m = __builtin_fmaxf(m, acc[r]);
+        }
+        if (!last) tile_lstore_padded<D, THREADS>(kb[(t + 1) & 1], SK, tid, kr);
+        __syncthreads();
+    }
+    m = __builtin_fmaxf(m, __shfl_xor(m, 32));
+    float ms;                                                   // the scaled maximum, with the sink
+    const RowExp ex(a, m, SINK, ms);
+
+    // pass 2: exponentials at the exact maximum, P.V with P = hi + lo
+    f32x16 o[D / 32];
+#pragma unroll
+    for (int dt = 0; dt < D / 32; dt++) o[dt] = f32x16{};
+    // the sink's exponential starts the row's sum (in one of its two lanes),
+    // so that nothing of it stays live across the tiles
+    float lsum = SINK && grp == 0 ? exp_poly(a.sink - ms) : 0.0f;
+    pv_walk<D, NW>(a, kg, vg, kb, vb, qb, ex, lim, nfull, 0, ntiles, tid, o, lsum);
     lsum += __shfl_xor(lsum, 32);
     if (rowv) {
         uint16_t *op = a.out + row * a.out_row + static_cast<uint64_t>(head) * D;
@@ -2152,7 +2199,7 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_attn(PrefillArgs a)
 // stages its own tiles (K rows padded to D + 8, V rows to D + 32) and loads
 // the next tile while computing this one.
 // ---------------------------------------------------------------------------
-template <int D, int KS, int TPW, bool POW2>
+template <int D, int KS, int TPW>
 __global__ __launch_bounds__(64 * KS, 1) void prefill_ks(PrefillArgs a)
 {
     constexpr int SK = Pad<D>::K, SV = Pad<D>::V;
@@ -2186,8 +2233,8 @@ __global__ __launch_bounds__(64 * KS, 1) void prefill_ks(PrefillArgs a)
     u32x4 kr[Tile<D, 64>::kPer], vr[Tile<D, 64>::kPer];
     tile_gload<D, 64, false>(kg, static_cast<uint64_t>(wave) * kKeyTile, a.n, l, kr);
 
-    // pass 1: the scores of this wave's tiles (unscaled dot products when
-    // POW2), kept, and their row maxima
+    // pass 1: the scores of this wave's tiles (unscaled dot products), kept,
+    // and their row maxima
     f32x16 sc[TPW];
     float m = kNegInf;
     {
@@ -2196,7 +2243,7 @@ __global__ __launch_bounds__(64 * KS, 1) void prefill_ks(PrefillArgs a)
 #pragma unroll
         for (int s = 0; s < D / 16; s++) {
             const u32x4 v = load16(qp + 16 * s + 8 * grp);
-            qb[s] = rowv ? v : u32x4{0, 0, 0, 0};
+            qb[s] = q_chunk(v, rowv, q_sign(a));
         }
         const int arow = swap23(col) * SK + 8 * grp;
 #pragma unroll
@@ -2227,14 +2274,12 @@ __global__ __launch_bounds__(64 * KS, 1) void prefill_ks(PrefillArgs a)
                 sc[i] = acc;
                 if (t < nfull) {
 #pragma unroll
-                    for (int r = 0; r < 16; r++) m = __builtin_fmaxf(m, POW2 ? acc[r] : acc[r] * a.scale);
+                    for (int r = 0; r < 16; r++) m = __builtin_fmaxf(m, acc[r]);
                 } else {
                     const int vis = static_cast<int>(static_cast<int64_t>(lim) - static_cast<int64_t>(t0));
 #pragma unroll
-                    for (int r = 0; r < 16; r++) {
-                        const float x = POW2 ? acc[r] : acc[r] * a.scale;
-                        if (key_of(r, grp) <= vis) m = __builtin_fmaxf(m, x);
-                    }
+                    for (int r = 0; r < 16; r++) 
+                        if (key_of(r, grp) <= vis) m = __builtin_fmaxf(m, acc[r]);
                 }
                 wave_sync();
             }
@@ -2249,11 +2294,8 @@ __global__ __launch_bounds__(64 * KS, 1) void prefill_ks(PrefillArgs a)
     for (int w = 0; w < KS; w++) m = __builtin_fmaxf(m, mred[w][col]);
     // rows past the chunk: a finite maximum, their outputs are never stored
     if (!rowv) m = 0.0f;
-    ExpArgs ex;
-    ex.m = m;
-    ex.scale = a.scale;
-    ex.clamp = POW2 ? -87.33654f / a.scale : -87.33654f;
-    ex.mul = POW2 ? 1.442695f * a.scale : 1.442695f;
+    float ms;
+    const RowExp ex(a, m, false, ms);
 
     // pass 2: exponentials of the kept scores at the exact maximum, P.V with
     // P = hi + lo
@@ -2281,7 +2323,7 @@ __global__ __launch_bounds__(64 * KS, 1) void prefill_ks(PrefillArgs a)
                 float ev[8];
 #pragma unroll
                 for (int r = 0; r < 8; r++) {
-                    const float e = exp_score<POW2>(sc[i][8 * h + r], ex);
+                    const float e = exp_score(sc[i][8 * h + r], ex);
                     ev[r] = full || key_of(8 * h + r, grp) <= vis ? e : 0.0f;
                     lsum += ev[r];
                 }
@@ -2412,7 +2454,7 @@ __device__ __forceinline__ void slice_mask_lstore(uint16_t *st, uint64_t t0, uin
     }
 }
 
-template <int D, int KS, int MT, int VPF, bool POW2>
+template <int D, int KS, int MT, int VPF>
 __global__ __launch_bounds__(64 * KS, 1) void prefill_kd(PrefillArgs a)
 {
     static_assert(KS == 4 || KS == 8, "a round's exponentials are spread over its tiles' products");
@@ -2471,13 +2513,13 @@ __global__ __launch_bounds__(64 * KS, 1) void prefill_kd(PrefillArgs a)
         for (int j = 0; j < QS; j++) {
             const int sq = wave * QS + j;
             const u32x4 v = load16(qp + 16 * sq + 8 * grp);
-            store16(qs + (sq * 64 + l) * 8, rowv ? v : u32x4{0, 0, 0, 0});
+            store16(qs + (sq * 64 + l) * 8, q_chunk(v, rowv, q_sign(a)));
         }
     }
     lds_barrier();
 
-    // pass 1: the scores of this wave's tiles (unscaled dot products when
-    // POW2), kept, and their row maxima
+    // pass 1: the scores of this wave's tiles (unscaled dot products), kept,
+    // and their row maxima
     f32x16 sc[TPW];
     float m = kNegInf;
     {
@@ -2516,10 +2558,7 @@ __global__ __launch_bounds__(64 * KS, 1) void prefill_kd(PrefillArgs a)
             const bool full = t < nfull;
             const int vis = static_cast<int>(static_cast<int64_t>(lim) - static_cast<int64_t>(t0));
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const float x = POW2 ? acc[r] : acc[r] * a.scale;
-                m = __builtin_fmaxf(m, full || key_of(r, grp) <= vis ? x : kNegInf);
-            }
+            for (int r = 0; r < 16; r++) m = __builtin_fmaxf(m, full || key_of(r, grp) <= vis ? acc[r] : kNegInf);
             wave_sync();
         }
     }
@@ -2536,11 +2575,8 @@ __global__ __launch_bounds__(64 * KS, 1) void prefill_kd(PrefillArgs a)
     for (int w = 0; w < KS; w++) m = __builtin_fmaxf(m, mred[w][col]);
     // rows past the chunk: a finite maximum, their outputs are never stored
     if (!rowv) m = 0.0f;
-    ExpArgs ex;
-    ex.m = m;
-    ex.scale = a.scale;
-    ex.clamp = POW2 ? -87.33654f / a.scale : -87.33654f;
-    ex.mul = POW2 ? 1.442695f * a.scale : 1.442695f;
+    float ms;
+    const RowExp ex(a, m, false, ms);
 
     // pass 2. exps_q(r, q): the exponentials of scores 4q .. 4q+3 of this
     // wave's tile of round r at the exact maximum, masked by bits (so that the
@@ -2554,7 +2590,7 @@ __global__ __launch_bounds__(64 * KS, 1) void prefill_kd(PrefillArgs a)
         const uint64_t t0 = static_cast<uint64_t>(t) * kKeyTile;
         const bool full = t < nfull;
         const int vis = static_cast<int>(static_cast<int64_t>(lim) - static_cast<int64_t>(t0));
-        const float e = exp_score<POW2>(sc[r][k], ex);
+        const float e = exp_score(sc[r][k], ex);
         const uint32_t keep = full || key_of(k, grp) <= vis ? 0xFFFFFFFFu : 0u;
         ev[k] = __uint_as_float(__float_as_uint(e) & keep);
         lsum += ev[k];
@@ -2756,7 +2792,7 @@ struct SplitSegs {
     }
 };
 
-template <int D, int HPW, bool POW2, int NW, bool PAIRED = false>
+template <int D, int HPW, int NW, bool PAIRED = false>
 __global__ __launch_bounds__(64 * NW, 1) void prefill_split_max(PrefillArgs a, SplitArgs sp)
 {
     constexpr int RB = NW / HPW, THREADS = 64 * NW;
@@ -2788,7 +2824,7 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_split_max(PrefillArgs a, S
 #pragma unroll
         for (int s = 0; s < D / 16; s++) {
             const u32x4 v = load16(qp + 16 * s + 8 * grp);
-            qb[s] = rowv ? v : u32x4{0, 0, 0, 0};
+            qb[s] = q_chunk(v, rowv, q_sign(a));
         }
         float m = kNegInf;
         if (tb < te) {
@@ -2812,14 +2848,12 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_split_max(PrefillArgs a, S
                 }
                 if (t < nfull) {
 #pragma unroll
-                    for (int r = 0; r < 16; r++) m = __builtin_fmaxf(m, POW2 ? acc[r] : acc[r] * a.scale);
+                    for (int r = 0; r < 16; r++) m = __builtin_fmaxf(m, acc[r]);
                 } else {
                     const int vis = static_cast<int>(static_cast<int64_t>(lim) - static_cast<int64_t>(t0));
 #pragma unroll
-                    for (int r = 0; r < 16; r++) {
-                        const float s = POW2 ? acc[r] : acc[r] * a.scale;
-                        if (key_of(r, grp) <= vis) m = __builtin_fmaxf(m, s);
-                    }
+                    for (int r = 0; r < 16; r++) 
+                        if (key_of(r, grp) <= vis) m = __builtin_fmaxf(m, acc[r]);
                 }
                 if (t + 1 < te) tile_lstore_padded<D, THREADS>(kb[(t - tb + 1) & 1], SK, tid, kr);
                 __syncthreads();
@@ -2833,10 +2867,10 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_split_max(PrefillArgs a, S
     if (PAIRED && segs.n > 1) run(segs.s1);
 }
 
-template <int D, int HPW, bool POW2, int NW, bool PAIRED = false, bool SINK = false>
+template <int D, int HPW, int NW, bool PAIRED = false, bool SINK = false>
 __global__ __launch_bounds__(64 * NW, 1) void prefill_split_pv(PrefillArgs a, SplitArgs sp)
 {
-    constexpr int RB = NW / HPW, THREADS = 64 * NW;
+    constexpr int RB = NW / HPW;
     constexpr int SK = Pad<D>::K, SV = Pad<D>::V;
     __shared__ __attribute__((aligned(16))) uint16_t kb[2][kKeyTile * SK];
     __shared__ __attribute__((aligned(16))) uint16_t vb[2][kKeyTile * SV];
@@ -2848,15 +2882,13 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_split_pv(PrefillArgs a, Sp
     const SplitSegs<PAIRED> segs(a, sid, 32 * RB);
     const uint16_t *kg = a.k + static_cast<uint64_t>(kvh) * a.kv_stride;
     const uint16_t *vg = a.v + static_cast<uint64_t>(kvh) * a.kv_stride;
-    const int arow = swap23(col) * SK + 8 * grp;
     auto run = [&](const SplitSeg sg, auto direct_t) {
         constexpr bool DIRECT = decltype(direct_t)::value;   // a whole row group: output written directly
         const uint64_t wg_r0 = static_cast<uint64_t>(sg.rg) * (32 * RB);
         const uint64_t w_r0 = wg_r0 + 32 * (wave / HPW);
         const uint64_t row = w_r0 + col;
         const bool rowv = row < a.rows;
-        const bool wact = w_r0 < a.rows;
-        const int nfull = wact ? static_cast<int>((a.past + w_r0 + 1) / kKeyTile) : 0;
+        const int nfull = w_r0 < a.rows ? static_cast<int>((a.past + w_r0 + 1) / kKeyTile) : 0;
         const uint64_t lim = a.past + row;
         const int tb = sg.tb, te = sg.te;
 
@@ -2869,21 +2901,15 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_split_pv(PrefillArgs a, Sp
             for (int z = 0; z < nz; z++)
                 m = __builtin_fmaxf(m, sp.smax[(static_cast<uint64_t>(z) * sp.heads + head) * a.rows + row]);
         }
-        float ms = 0.0f;                                        // the scaled maximum, with the sink
-        if constexpr (SINK) m = sink_max<POW2>(m, a, ms);
-        ExpArgs ex;
-        ex.m = m;
-        ex.scale = a.scale;
-        ex.clamp = POW2 ? -87.33654f / a.scale : -87.33654f;
-        ex.mul = POW2 ? 1.442695f * a.scale : 1.442695f;
+        float ms;                                                   // the scaled maximum, with the sink
+        const RowExp ex(a, m, SINK, ms);
 
-        u32x4 kr[Tile<D, THREADS>::kPer], vr[Tile<D, THREADS>::kPer];
         u32x4 qb[D / 16];
         const uint16_t *qp = a.q + (rowv ? row : 0) * a.q_row + static_cast<uint64_t>(head) * a.q_head;
 #pragma unroll
         for (int s = 0; s < D / 16; s++) {
             const u32x4 v = load16(qp + 16 * s + 8 * grp);
-            qb[s] = rowv ? v : u32x4{0, 0, 0, 0};
+            qb[s] = q_chunk(v, rowv, q_sign(a));
         }
         f32x16 o[D / 32];
 #pragma unroll
@@ -2891,69 +2917,7 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_split_pv(PrefillArgs a, Sp
         // the sink's exponential, once per row: it starts the sum of the whole
         // range's or of slot 0's (in one lane of two)
         float lsum = SINK && (DIRECT || sg.slot == 0) && grp == 0 ? exp_poly(a.sink - ms) : 0.0f;
-        if (tb < te) {
-            tile_gload<D, THREADS, false>(kg, static_cast<uint64_t>(tb) * kKeyTile, a.n, tid, kr);
-            tile_gload<D, THREADS, false>(vg, static_cast<uint64_t>(tb) * kKeyTile, a.n, tid, vr);
-            tile_lstore_padded<D, THREADS>(kb[0], SK, tid, kr);
-            tile_mask<D, THREADS>(static_cast<uint64_t>(tb) * kKeyTile, a.n, tid, vr);
-            tile_lstore_padded<D, THREADS>(vb[0], SV, tid, vr);
-            __syncthreads();
-            // as prefill_attn's pass 2: loads not branched around, the masked
-            // and unmasked halves of a tile instantiated apart, the P.V MFMAs
-            // at raised priority
-            for (int t = tb; t < te; t++) {
-                const uint64_t t0 = static_cast<uint64_t>(t) * kKeyTile;
-                const int b = (t - tb) & 1;
-                tile_gload<D, THREADS, false>(kg, t0 + kKeyTile, a.n, tid, kr);  // past the cache: row 0, unused
-                __builtin_amdgcn_sched_barrier(0);
-                f32x16 acc = {};
-#pragma unroll
-                for (int s = 0; s < D / 16; s += 2) {
-                    // two K operands requested before their MFMAs
-                    const u32x4 k0 = load16(kb[b] + arow + 16 * s), k1 = load16(kb[b] + arow + 16 * (s + 1));
-                    acc = mfma(k0, qb[s], acc);
-                    acc = mfma(k1, qb[s + 1], acc);
-                }
-                const bool full = t < nfull;
-                const int vis = static_cast<int>(static_cast<int64_t>(lim) - static_cast<int64_t>(t0));
-                auto half = [&](int h, auto masked, u32x4 &hi, u32x4 &lo) {
-                    constexpr bool MASKED = decltype(masked)::value;
-                    float ev[8];
-#pragma unroll
-                    for (int r = 0; r < 8; r++) {
-                        const float e = exp_score<POW2>(acc[8 * h + r], ex);
-                        ev[r] = !MASKED || key_of(8 * h + r, grp) <= vis ? e : 0.0f;
-                        lsum += ev[r];
-                    }
-                    split_pack_hw(ev, hi, lo);
-                };
-                auto pv = [&](int h, const u32x4 &hi, const u32x4 &lo) {
-                    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-                    for (int dt = 0; dt < D / 32; dt++) {
-                        const u32x4 av = vt_operand_padded<D>(vb[b], 16 * h, 32 * dt, l);
-                        o[dt] = mfma(av, hi, o[dt]);
-                        o[dt] = mfma(av, lo, o[dt]);
-                    }
-                    __builtin_amdgcn_s_setprio(0);
-                };
-                u32x4 hi, lo;
-                if (full) half(0, std::false_type{}, hi, lo);
-                else half(0, std::true_type{}, hi, lo);
-                tile_gload<D, THREADS, false>(vg, t0 + kKeyTile, a.n, tid, vr);
-                __builtin_amdgcn_sched_barrier(0);
-                pv(0, hi, lo);
-                if (full) half(1, std::false_type{}, hi, lo);
-                else half(1, std::true_type{}, hi, lo);
-                pv(1, hi, lo);
-                if (t + 1 < te) {
-                    tile_lstore_padded<D, THREADS>(kb[b ^ 1], SK, tid, kr);
-                    tile_mask<D, THREADS>(t0 + kKeyTile, a.n, tid, vr);
-                    tile_lstore_padded<D, THREADS>(vb[b ^ 1], SV, tid, vr);
-                }
-                __syncthreads();
-            }
-        }
+        if (tb < te) pv_walk<D, NW>(a, kg, vg, kb, vb, qb, ex, lim, nfull, tb, te, tid, o, lsum);
         lsum += __shfl_xor(lsum, 32);
         if (!rowv) return;
         if constexpr (DIRECT) {
@@ -2998,32 +2962,15 @@ template <int D>
 __global__ __launch_bounds__(CombineShape<D>::THREADS) void prefill_split_combine_wide(PrefillArgs a, SplitArgs sp,
                                                                                        int splits);
 
-// A positive power of two in [2^-20, 2^20]: scaling by it is exact for the
-// scores and for the folded exponential constants.
-static bool scale_is_pow2(float s)
-{
-    const uint32_t b = __builtin_bit_cast(uint32_t, s);
-    const uint32_t e = (b >> 23) & 0xFF;
-    return (b & 0x807FFFFFu) == 0 && e >= 127 - 20 && e <= 127 + 20;
-}
-
-// The three split kernels on grid (row groups, head groups, splits). POW2:
-// whether a power-of-two scale takes the folded form (the general form rounds
-// identically).
-template <int D, int HPW, int NW, bool POW2_FORM = true, bool SINK = false>
+// The three split kernels on grid (row groups, head groups, splits).
+template <int D, int HPW, int NW, bool SINK = false>
 static hipError_t launch_prefill_split(const PrefillArgs &a, int heads, const PrefillSplit &ps, dim3 grid, int splits,
                                        hipStream_t s)
 {
     const SplitArgs sp{ps.smax, ps.so, ps.sl, heads, 0, a.rows};
     const dim3 gs(grid.x, grid.y, static_cast<unsigned>(splits));
-    hipError_t e;
-    if (POW2_FORM && scale_is_pow2(a.scale)) {
-        e = launch(prefill_split_max<D, HPW, POW2_FORM, NW>, gs, dim3(64 * NW), s, a, sp);
-        if (e == hipSuccess) e = launch(prefill_split_pv<D, HPW, POW2_FORM, NW, false, SINK>, gs, dim3(64 * NW), s, a, sp);
-    } else {
-        e = launch(prefill_split_max<D, HPW, false, NW>, gs, dim3(64 * NW), s, a, sp);
-        if (e == hipSuccess) e = launch(prefill_split_pv<D, HPW, false, NW, false, SINK>, gs, dim3(64 * NW), s, a, sp);
-    }
+    hipError_t e = launch(prefill_split_max<D, HPW, NW>, gs, dim3(64 * NW), s, a, sp);
+    if (e == hipSuccess) e = launch(prefill_split_pv<D, HPW, NW, false, SINK>, gs, dim3(64 * NW), s, a, sp);
     if (e != hipSuccess) return e;
     const dim3 gc(static_cast<unsigned>(a.rows), heads);
     return splits > kCombineNarrowSplits
@@ -3033,7 +2980,7 @@ static hipError_t launch_prefill_split(const PrefillArgs &a, int heads, const Pr
 
 // The paired form on the causal kernel's grid (row groups, head groups); pr
 // from prefill_pairs.
-template <int D, int HPW, int NW, bool POW2_FORM = true, bool SINK = false>
+template <int D, int HPW, int NW, bool SINK = false>
 static hipError_t launch_prefill_paired(const PrefillArgs &a, int heads, const PrefillSplit &ps, dim3 grid,
                                         const PairRows &pr, hipStream_t s)
 {
@@ -3043,15 +2990,8 @@ static hipError_t launch_prefill_paired(const PrefillArgs &a, int heads, const P
     // waves per SIMD, where the pairs' one per CU left the K operand reads'
     // latency exposed; the P.V pass takes the larger of the two
     const dim3 gmax(grid.x, grid.y, 2);
-    hipError_t e;
-    if (POW2_FORM && scale_is_pow2(a.scale)) {
-        e = launch(prefill_split_max<D, HPW, POW2_FORM, NW, false>, gmax, dim3(64 * NW), s, a, sp);
-        if (e == hipSuccess)
-            e = launch(prefill_split_pv<D, HPW, POW2_FORM, NW, true, SINK>, grid, dim3(64 * NW), s, a, sp);
-    } else {
-        e = launch(prefill_split_max<D, HPW, false, NW, false>, gmax, dim3(64 * NW), s, a, sp);
-        if (e == hipSuccess) e = launch(prefill_split_pv<D, HPW, false, NW, true, SINK>, grid, dim3(64 * NW), s, a, sp);
-    }
+    hipError_t e = launch(prefill_split_max<D, HPW, NW>, gmax, dim3(64 * NW), s, a, sp);
+    if (e == hipSuccess) e = launch(prefill_split_pv<D, HPW, NW, true, SINK>, grid, dim3(64 * NW), s, a, sp);
     if (e != hipSuccess) return e;
     return launch(prefill_split_combine<D>, dim3(static_cast<unsigned>(pr.srows), heads), dim3(D), s, a, sp, 2);
 }

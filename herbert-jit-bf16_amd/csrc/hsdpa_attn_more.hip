@@ -5,9 +5,7 @@
 // the tuned instantiations there are compiled exactly as before.
 //
 // Configurations: the causal kernel serves one query head per workgroup
-// (HPW = 1, valid for every group size) and always scales the scores first
-// (the general path; with a power-of-two scale it rounds identically to the
-// folded one). Up to D = 256 it runs 8 waves, two per SIMD; above, the O and
+// (HPW = 1, valid for every group size). Up to D = 256 it runs 8 waves, two per SIMD; above, the O and
 // Q registers of a 32-row wave (D/2 + D/4) exceed the 256 of two waves per
 // SIMD, so it runs 4 waves, one per SIMD. The decode passes take the
 // configurations decode_loop_ok / decode_wide_ok allow.
@@ -52,10 +50,10 @@ static hipError_t prefill_more_d(const PrefillArgs &a, int heads, const PrefillS
     constexpr int ROWS = 32 * NW;                                // HPW = 1: NW row blocks of one head
     const dim3 grid(static_cast<unsigned>((a.rows + ROWS - 1) / ROWS), heads);
     const int splits = prefill_splits(a, static_cast<uint64_t>(grid.x) * grid.y, heads, ps);
-    if (splits > 1) return launch_prefill_split<D, 1, NW, false>(a, heads, ps, grid, splits, s);
+    if (splits > 1) return launch_prefill_split<D, 1, NW>(a, heads, ps, grid, splits, s);
     const PairRows pr = prefill_pairs(a, grid.x, static_cast<uint64_t>(grid.x) * grid.y, ROWS, heads, ps);
-    if (pr.srows) return launch_prefill_paired<D, 1, NW, false>(a, heads, ps, grid, pr, s);
-    return launch(prefill_attn<D, 1, false, NW>, grid, dim3(64 * NW), s, a);
+    if (pr.srows) return launch_prefill_paired<D, 1, NW>(a, heads, ps, grid, pr, s);
+    return launch(prefill_attn<D, 1, NW>, grid, dim3(64 * NW), s, a);
 }
 
 #define HSDPA_MORE_DIMS(X) \

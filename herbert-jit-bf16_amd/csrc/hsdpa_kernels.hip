@@ -409,8 +409,7 @@ static hipError_t prefill_dh(const PrefillArgs &a, int heads, const PrefillSplit
     if (splits > 1) return launch_prefill_split<D, HPW, 8>(a, heads, ps, grid, splits, s);
     const PairRows pr = prefill_pairs(a, grid.x, static_cast<uint64_t>(grid.x) * grid.y, 32 * (8 / HPW), heads, ps);
     if (pr.srows) return launch_prefill_paired<D, HPW, 8>(a, heads, ps, grid, pr, s);
-    if (scale_is_pow2(a.scale)) return launch(prefill_attn<D, HPW, true>, grid, dim3(512), s, a);
-    return launch(prefill_attn<D, HPW, false>, grid, dim3(512), s, a);
+    return launch(prefill_attn<D, HPW>, grid, dim3(512), s, a);
 }
 
 template <int D>

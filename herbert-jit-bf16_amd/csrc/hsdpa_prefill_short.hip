@@ -8,15 +8,15 @@
 
 namespace hsdpa {
 
-template <int D, int MT, bool POW2, int KS = kShortWaves>
+template <int D, int MT, int KS = kShortWaves>
 static hipError_t prefill_kd_mt(const PrefillArgs &a, int heads, hipStream_t s)
 {
     const dim3 grid(static_cast<unsigned>((a.rows + 31) / 32), static_cast<unsigned>(heads));
-    return launch(prefill_kd<D, KS, MT, 4, POW2>, grid, dim3(64 * KS), s, a);
+    return launch(prefill_kd<D, KS, MT, 4>, grid, dim3(64 * KS), s, a);
 }
 
-template <int D, bool POW2>
-static hipError_t prefill_short_dp(const PrefillArgs &a, int heads, hipStream_t s)
+template <int D>
+static hipError_t prefill_short_d(const PrefillArgs &a, int heads, hipStream_t s)
 {
     const uint64_t ntiles = (a.past + a.rows + kKeyTile - 1) / kKeyTile;
     // D = 128 and 256: O by dimensions, no partial outputs between the waves,
@@ -33,24 +33,18 @@ static hipError_t prefill_short_dp(const PrefillArgs &a, int heads, hipStream_t 
     // 14.8 against 4 waves. D = 64: O by keys.
     if constexpr (D == 64) {
         const dim3 grid(static_cast<unsigned>((a.rows + 31) / 32), static_cast<unsigned>(heads));
-        return launch(prefill_ks<D, kShortWaves, kShortMaxTiles / kShortWaves, POW2>, grid, dim3(64 * kShortWaves),
+        return launch(prefill_ks<D, kShortWaves, kShortMaxTiles / kShortWaves>, grid, dim3(64 * kShortWaves),
                       s, a);
     } else {
         constexpr int KS = D == 256 ? 8 : kShortWaves;
-        if (ntiles <= 8) return prefill_kd_mt<D, 8, POW2, KS>(a, heads, s);
+        if (ntiles <= 8) return prefill_kd_mt<D, 8, KS>(a, heads, s);
         if constexpr (D == 128)
-            if (ntiles <= 12) return prefill_kd_mt<D, 12, POW2, KS>(a, heads, s);
-        if (ntiles <= 16) return prefill_kd_mt<D, 16, POW2, KS>(a, heads, s);
-        if (ntiles <= 24) return prefill_kd_mt<D, 24, POW2, KS>(a, heads, s);
-        if (ntiles <= static_cast<uint64_t>(kShortMaxTiles)) return prefill_kd_mt<D, 32, POW2, KS>(a, heads, s);
+            if (ntiles <= 12) return prefill_kd_mt<D, 12, KS>(a, heads, s);
+        if (ntiles <= 16) return prefill_kd_mt<D, 16, KS>(a, heads, s);
+        if (ntiles <= 24) return prefill_kd_mt<D, 24, KS>(a, heads, s);
+        if (ntiles <= static_cast<uint64_t>(kShortMaxTiles)) return prefill_kd_mt<D, 32, KS>(a, heads, s);
         return hipErrorInvalidValue;
     }
-}
-
-template <int D>
-static hipError_t prefill_short_d(const PrefillArgs &a, int heads, hipStream_t s)
-{
-    return scale_is_pow2(a.scale) ? prefill_short_dp<D, true>(a, heads, s) : prefill_short_dp<D, false>(a, heads, s);
 }
 
 hipError_t launch_prefill_short(const PrefillArgs &a, int head_dim, int heads, hipStream_t s)

@@ -9,7 +9,7 @@
 //
 // The kernels are prefill_attn and the split pair of hsdpa_attn_kernels.h with
 // SINK set: one query head per workgroup (HPW = 1, valid for every group
-// size), the scores scaled first (the general path), 8 waves up to D = 256 and
+// size), 8 waves up to D = 256 and
 // 4 above, as hsdpa_attn_more.hip configures the other head dimensions. The
 // short-chunk kernels are not instantiated with the sink: such chunks take
 // these. In a translation unit of its own, so that the kernels without the
@@ -26,10 +26,10 @@ static hipError_t prefill_sink_d(const PrefillArgs &a, int heads, const PrefillS
     constexpr int ROWS = 32 * NW;                                // NW row blocks of one head
     const dim3 grid(static_cast<unsigned>((a.rows + ROWS - 1) / ROWS), heads);
     const int splits = prefill_splits(a, static_cast<uint64_t>(grid.x) * grid.y, heads, ps);
-    if (splits > 1) return launch_prefill_split<D, 1, NW, false, true>(a, heads, ps, grid, splits, s);
+    if (splits > 1) return launch_prefill_split<D, 1, NW, true>(a, heads, ps, grid, splits, s);
     const PairRows pr = prefill_pairs(a, grid.x, static_cast<uint64_t>(grid.x) * grid.y, ROWS, heads, ps);
-    if (pr.srows) return launch_prefill_paired<D, 1, NW, false, true>(a, heads, ps, grid, pr, s);
-    return launch(prefill_attn<D, 1, false, NW, true>, grid, dim3(64 * NW), s, a);
+    if (pr.srows) return launch_prefill_paired<D, 1, NW, true>(a, heads, ps, grid, pr, s);
+    return launch(prefill_attn<D, 1, NW, true>, grid, dim3(64 * NW), s, a);
 }
 
 #define HSDPA_SINK_DIMS(X)                                                                                  \
