@@ -381,31 +381,24 @@ DecodeCfg decode_cfg(const hsdpa_plan *p, uint64_t rows, uint64_t n, int sub, bo
         const uint64_t tiles = (n + hsdpa::kKeyTile - 1) / hsdpa::kKeyTile;
         const uint64_t run = hsdpa::kKeyTile * ((tiles + per - 1) / per);
         c.keys_pv = groups * nch <= cu1 || !hsdpa::decode_pv_loop_ok(d, c.g, static_cast<int>(rows), fused) ||
-                            !hsdpa::decode_pv_loop_rows_ok(d, static_cast<int>(rows), sub, p->kv_heads * nch, cu1) ||
                             run > (1u << 30)
                         ? hsdpa::kDecodeKeysPV
                         : static_cast<int>(run);
     }
-    // a few rows at D = 256 in 2 to 4 groups where pass 1 takes all of a KV
-    // head's groups and 256-key workgroups would take more than one round:
-    // one round of workgroups that each walk a run for all the groups
-    // (decode_pv_all_loop_ok), the CUs shared among the KV heads only
-    bool all_loop = false;
-    if (!fused && hsdpa::decode_pv_all_loop_ok(d, static_cast<int>(rows), sub, c.qk_all != 0, p->kv_heads * nch, cu1)) {
-        const uint64_t per = cu1 / p->kv_heads > 0 ? cu1 / p->kv_heads : 1;
+    // D = 256, past one round of 256-key workgroups per group: pass 2 takes all
+    // the groups of a KV head in each workgroup, in one round of runs of whole
+    // tiles (decode_pv_groups_ok)
+    if (!fused && groups * nch > cu1) {
+        const uint64_t per = hsdpa::decode_pv_groups_wgs(p->kv_heads, cu1);
         const uint64_t tiles = (n + hsdpa::kKeyTile - 1) / hsdpa::kKeyTile;
-        const uint64_t run = hsdpa::kKeyTile * ((tiles + per - 1) / per);
-        if (run > static_cast<uint64_t>(hsdpa::kDecodeKeysPV) && run <= (uint64_t{1} << 30)) {
-            c.keys_pv = static_cast<int>(run);
-            all_loop = true;
+        const uint64_t run = std::max<uint64_t>((tiles + per - 1) / per, 4);
+        if (hsdpa::decode_pv_groups_ok(d, sub, c.g, run)) {
+            c.keys_pv = static_cast<int>(run) * hsdpa::kKeyTile;
+            c.pv_all = 1;
         }
     }
     c.nwg_qk = static_cast<int>((n + c.keys_qk - 1) / c.keys_qk);
     c.nwg_pv = static_cast<int>((n + c.keys_pv - 1) / c.keys_pv);
-    // where pass 1 takes all of a KV head's groups and pass 2 runs 256-key
-    // workgroups (D = 256; at D = 64 and 128 it takes chunks there), pass 2
-    // takes them all too: each V tile loaded once instead of once per group
-    c.pv_all = (c.qk_all && c.keys_pv == hsdpa::kDecodeKeysPV && d == 256) || all_loop ? 1 : 0;
     // a short cache: pass 2 writes the outputs itself, no combine launch
     c.direct = hsdpa::decode_direct_ok(d, static_cast<int>(rows), sub, c.g, n, fused) ? 1 : 0;
     // several groups: a key range's groups on one XCD, whose L2 then serves
@@ -431,6 +424,14 @@ uint64_t decode_nwg_pv_max(const hsdpa_plan *p, uint64_t rows, int sub)
     const int g = hsdpa::decode_group_cols(static_cast<int>(rows * p->spec.gqa), sub);
     if (!hsdpa::decode_wide_ok(d)) return by128;
     const uint64_t one_round = std::min(by128, per);
+    // all groups per workgroup (the Chained rows): one round of them, at least
+    // 128 keys each
+    uint64_t all = 0;
+    const uint64_t per_all = hsdpa::decode_pv_groups_wgs(p->kv_heads, static_cast<uint64_t>(p->cus));
+    if (hsdpa::decode_pv_groups_dim(d, sub)) {
+        all = std::min(by128, per_all);
+        if (p->form != HSDPA_FORM_FUSED && (sub > 1 || g > 8)) return all;
+    }
     // the chunked pass 2 gives way to 256-key workgroups where it cannot run
     // (decode_pv_loop_ok) or a run would exceed 2^30 keys
     const uint64_t run_max = 32 * (((cap + 31) / 32 + per - 1) / per);
@@ -438,15 +439,8 @@ uint64_t decode_nwg_pv_max(const hsdpa_plan *p, uint64_t rows, int sub)
     const bool loop = hsdpa::decode_pv_loop_ok(d, g, static_cast<int>(rows), false) &&
                       (p->form != HSDPA_FORM_FUSED || hsdpa::decode_pv_loop_ok(d, g, static_cast<int>(rows), true));
     if (!loop || run_max > (uint64_t{1} << 30))
-        return std::max(one_round, by256);
-    // several rows at D = 256: 256-key workgroups where decode_pv_loop_rows_ok
-    // declines the runs (for any past with more than 4 groups; up to
-    // CUs / kv_heads of them where they fit one round)
-    if (d == 256 && rows > 1 && sub > 1) {
-        if (sub > 4) return std::max(one_round, by256);
-        return std::max(one_round, std::min(by256, static_cast<uint64_t>(p->cus) / p->kv_heads));
-    }
-    return one_round;
+        return std::max({all, one_round, by256});
+    return std::max(all, one_round);
 }
 
 // The Fused form's rows outside full chunks of 8: the last rows % 8 (the

@@ -98,6 +98,50 @@ __device__ __forceinline__ uint32_t cvt_out(float x)
     return e == 0 ? ((b >> 16) & 0x8000u) : r;
 }
 
+// One row's exponential: see exp_score. From x's exponent t = x c + b.
+struct RowExp {
+    float c, b;
+    // The exponential of x - X where X has the exponent X xc (xc = c, or the
+    // scaled maximum's own factor). Where the exponent of the maximum itself
+    // would leave the f32 range, two scores that differ at all differ by far
+    // more than the exponential's clamp, and a smaller c tells them apart as
+    // well.
+    __device__ __forceinline__ RowExp(float cc, float X, float xc)
+    {
+        c = cc;
+        float t = X * xc;
+        if (__builtin_fabsf(t) > 1e38f) {
+            c *= 0x1p-24f;
+            t = X * (xc * 0x1p-24f);
+        }
+        b = 0.5f - t;
+    }
+    // of scaled scores, m their maximum
+    __device__ __forceinline__ explicit RowExp(float m) : RowExp(1.442695f, m, 1.442695f) {}
+};
+
+// P(x - M) of the score x (acc: x or its dot product): t = (x - M) log2(e) + 1/2
+// in one rounding, clamped as the emitted exponential clamps (a NaN too), k =
+// floor(t), and the emitted polynomial about t - k - 1/2, its argument moved
+// by 1/2 into the coefficients: P(x) 2^k = Q(t - k) 2^k. Nine instructions
+// where subtract, clamp, scale, round, subtract, convert, polynomial and
+// ldexp take eleven (and one more for a scale that is no power of two): the
+// causal passes are VALU-bound up to D = 128. Against 64-bit exponentials over
+// |score - M| up to 30, relative rms 1.42e-5 and largest 6.1e-5, both the
+// polynomial's own and the same either way.
+__device__ __forceinline__ float exp_score(float acc, const RowExp &x)
+{
+    const float t = __builtin_fmaxf(__builtin_fmaf(acc, x.c, x.b), -125.49977f);
+    int k;
+    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(k) : "v"(t));
+    const float f = __builtin_amdgcn_fractf(t);
+    float p = __builtin_fmaf(f, 0.00967248f, 0.03615915f);
+    p = __builtin_fmaf(f, p, 0.17147906f);
+    p = __builtin_fmaf(f, p, 0.4897125f);
+    p = __builtin_fmaf(f, p, 0.70714957f);
+    return __builtin_ldexpf(p, k);
+}
+
 // The output gate of one element (ElemOp::SigmoidMul, emit_elem.rs:350-440):
 // e = 0 - g; e = e < 88 ? e : 88 (vminps: the bound when e is NaN); the
 // softmax's exponential; bf16(a / (e + 1)), a the bf16 attention output.
@@ -1167,378 +1211,235 @@ __global__ __launch_bounds__(64 * W, D > 256 ? 1 : 8 / W) void decode_pv(DecodeA
 }
 
 // ---------------------------------------------------------------------------
-// Decode pass 2 over every group of a KV head in one workgroup (2 to
-// kDecodeMaxSub groups of 9 to 16 columns; 8 waves, 256 keys, as decode_pv's
-// 8-wave form with two P column blocks). The V tiles are loaded and staged in
-// LDS once, and each wave reads its V^T operands into registers once; then,
-// for each group in turn, the exact maximum of its columns, the exponentials
-// (hi + lo P columns in LDS) and P.V, the scores and maxima of the group
-// after next requested before this group's products (two groups in flight). The partials go where decode_pv
-// puts them, so the combine is the same. Every column carries its row's
-// causal limit (a few rows; one row sees all keys). Grid (nwg_pv, kv_heads).
-// ---------------------------------------------------------------------------
-template <int D>
-__global__ __launch_bounds__(512, 1) void decode_pv_all(DecodeArgs a)
-{
-    constexpr int W = 8, NCB = 2, THREADS = 64 * W, KEYS = W * kKeyTile, PS = KEYS + 8;
-    constexpr int DB = D / 16, DBW = DB / W, nh = 8 * NCB;
-    static_assert(DB % W == 0, "each wave takes whole dimension blocks");
-    constexpr int T = THREADS / nh, BATCH = 8;                  // lanes per column's maxima
-    __shared__ __attribute__((aligned(16))) uint16_t vt[W][kKeyTile * D];
-    __shared__ __attribute__((aligned(16))) uint16_t pc[2 * kDecodeMaxGroup * PS];
-    __shared__ float smax[kDecodeMaxGroup];
-    __shared__ float lpart[W][kDecodeMaxGroup];
-    const int wg = static_cast<int>(blockIdx.x), tid = threadIdx.x;
-    const int kvh0 = static_cast<int>(blockIdx.y) * a.sub, ng = a.sub;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, j = l & 15, G = l >> 4;
-    const uint64_t j0 = static_cast<uint64_t>(wg) * KEYS;
-    const uint64_t j1 = j0 + KEYS < a.n ? j0 + KEYS : a.n;
-    const uint16_t *vbase = a.v + static_cast<uint64_t>(blockIdx.y) * a.kv_stride;
-    const int key_e = tid % KEYS;
-    const uint64_t gk = j0 + key_e;
-    const bool kv_e = gk < j1;
-    const int jh = tid / T, u = tid % T;
-    // two groups' loads in flight: group z's scores and maxima arrive while
-    // group z - 1 is computed (buffer z % 2)
-    float sva[kDecodeMaxGroup / 2], mxa[BATCH], svb[kDecodeMaxGroup / 2], mxb[BATCH];
-    const int hq = __builtin_amdgcn_readfirstlane(tid / KEYS);  // the same in a whole wave
-    // group z's scores of this thread's key (columns hq + 2 i, whose addresses
-    // are the same in a whole wave) and the first batch of its columns'
-    // pass-1 maxima
-    auto load_group = [&](int z, float(&sv)[kDecodeMaxGroup / 2], float(&mx)[BATCH]) {
-        const int kvh = kvh0 + z;
-        const uint64_t key = kv_e ? gk : 0;
-#pragma unroll
-        for (int i = 0; i < nh / 2; i++) {
-            const int h = hq + 2 * i;
-            const float *col = a.scores + static_cast<uint64_t>(kvh * a.g + (h < a.g ? h : 0)) * a.npad;
-            sv[i] = col[key];
-        }
-        const float *msrc = a.wgmax + (static_cast<uint64_t>(kvh) * a.g + (jh < a.g ? jh : 0)) * a.nwg_qk;
-#pragma unroll
-        for (int b = 0; b < BATCH; b++) {
-            const int w = u + b * T;
-            mx[b] = msrc[w < a.nwg_qk ? w : 0];
-        }
-    };
-    load_group(0, sva, mxa);
-    if (ng > 1) load_group(1, svb, mxb);
-    u32x4 vr[Tile<D, 64>::kPer];
-    tile_gload<D, 64, true>(vbase, j0 + kKeyTile * wave, j1, l, vr);
-    __builtin_amdgcn_sched_barrier(0);                          // all loads issued first
-    u32x4 av[W][DBW];                                           // this wave's V^T operands, all tiles
-    // one group: FIRST also stages V and reads the V^T operands; ODD takes
-    // buffer b
-    auto group = [&](int z, auto first_t, auto odd_t) {
-        constexpr bool FIRST = decltype(first_t)::value, ODD = decltype(odd_t)::value;
-        float(&sv)[kDecodeMaxGroup / 2] = ODD ? svb : sva;
-        float(&mx)[BATCH] = ODD ? mxb : mxa;
-        const int kvh = kvh0 + z;
-        float m = kNegInf;
-#pragma unroll
-        for (int b = 0; b < BATCH; b++) m = (u + b * T < a.nwg_qk && mx[b] > m) ? mx[b] : m;
-        const float *msrc = a.wgmax + (static_cast<uint64_t>(kvh) * a.g + (jh < a.g ? jh : 0)) * a.nwg_qk;
-        for (int w0 = u + BATCH * T; w0 < a.nwg_qk; w0 += BATCH * T) {
-#pragma unroll
-            for (int b = 0; b < BATCH; b++) {
-                const int w = w0 + b * T;
-                mx[b] = msrc[w < a.nwg_qk ? w : 0];
-            }
-#pragma unroll
-            for (int b = 0; b < BATCH; b++) m = (w0 + b * T < a.nwg_qk && mx[b] > m) ? mx[b] : m;
-        }
-        m = group_max_hi(m, T);
-        if (a.sink_on) m = m > a.sink ? m : a.sink;             // the sink joins the maximum
-        // the previous group's P operand reads and partial sums are done
-        // before this barrier, so its slots may be rewritten after it
-        if (u == T - 1 && jh < a.g) smax[jh] = m;
-        __syncthreads();
-        // column tid's maximum, for the sink's term (smax is rewritten by the
-        // next group once every wave has passed this group's second barrier)
-        const float mcol = tid < a.g ? smax[tid] : 0.0f;
-        // every column slot at once, with no branch between them (as in
-        // decode_pv); slots past g get zeros
-        float ev[nh / 2];
-        // column h's row sees keys [0, past + row], row = (z g + h) / G, by
-        // steps of two columns
-        ColumnRows rows(z * a.g + hq, a.G);
-#pragma unroll
-        for (int i = 0; i < nh / 2; i++) {
-            const int h = hq + 2 * i;
-            if (i > 0) rows.next2();
-            const bool vis = (h < a.g) & kv_e & (gk <= a.past + static_cast<uint64_t>(rows.row));
-            const float x = exp_poly(sv[i] - smax[h]);          // computed in every lane, then selected
-            ev[i] = vis ? x : 0.0f;
-        }
-#pragma unroll
-        for (int i = 0; i < nh / 2; i += 2) {
-            const int h = hq + 2 * i;                           // slots i and i + 1: columns h, h + 2
-            uint32_t hb, lb;
-            split2(ev[i], ev[i + 1], hb, lb);
-            pc[h * PS + key_e] = static_cast<uint16_t>(hb);
-            pc[(h + 2) * PS + key_e] = static_cast<uint16_t>(hb >> 16);
-            pc[(nh + h) * PS + key_e] = static_cast<uint16_t>(lb);
-            pc[(nh + h + 2) * PS + key_e] = static_cast<uint16_t>(lb >> 16);
-        }
-        float esum[nh / 2];
-#pragma unroll
-        for (int i = 0; i < nh / 2; i++) esum[i] = wave_sum_hi(ev[i]);
-        if (l == 63) {
-#pragma unroll
-            for (int i = 0; i < nh / 2; i++) lpart[wave][hq + 2 * i] = esum[i];
-        }
-        if (z + 2 < ng) load_group(z + 2, sv, mx);
-        if constexpr (FIRST) tile_mask_lstore_v16<D, 64>(vt[wave], j0 + kKeyTile * wave, j1, l, vr);
-        __syncthreads();
-        if constexpr (FIRST) {
-#pragma unroll
-            for (int t = 0; t < W; t++)
-#pragma unroll
-                for (int db = 0; db < DBW; db++) av[t][db] = vt16_operand<D>(vt[t], 16 * (wave * DBW + db), l);
-        }
-        u32x4 bp[W][NCB];
-#pragma unroll
-        for (int t = 0; t < W; t++)
-#pragma unroll
-            for (int c = 0; c < NCB; c++) bp[t][c] = load16(pc + (16 * c + j) * PS + kKeyTile * t + 8 * G);
-        __builtin_amdgcn_sched_barrier(0);
-        f32x4 o[NCB][DBW] = {};
-#pragma unroll
-        for (int t = 0; t < W; t++)
-#pragma unroll
-            for (int db = 0; db < DBW; db++)
-#pragma unroll
-                for (int c = 0; c < NCB; c++) o[c][db] = mfma16(av[t][db], bp[t][c], o[c][db]);
-        // O(column) = O(hi block) + O(lo block)
-        const uint64_t pbase = (static_cast<uint64_t>(kvh) * a.nwg_pv + wg) * a.g;
-#pragma unroll
-        for (int db = 0; db < DBW; db++) {
-            if (j < a.g) {
-                float *dst = a.part_o + (pbase + j) * D + 16 * (wave * DBW + db) + 4 * G;
-                *reinterpret_cast<float4 *>(dst) = float4{o[0][db][0] + o[1][db][0], o[0][db][1] + o[1][db][1],
-                                                          o[0][db][2] + o[1][db][2], o[0][db][3] + o[1][db][3]};
-            }
-        }
-        if (tid < a.g) {
-            // columns of parity p were summed by waves 4 p .. 4 p + 3, 64 keys each
-            const int p0 = (tid % (THREADS / KEYS)) * (KEYS / 64);
-            float L = 0.0f;
-            for (int w = 0; w < KEYS / 64; w++) L += lpart[p0 + w][tid];
-            if (a.sink_on && wg == 0) L += exp_poly(a.sink - mcol);  // once per column
-            a.part_l[pbase + tid] = L;
-        }
-    };
-    group(0, std::true_type{}, std::false_type{});
-    for (int z = 1; z < ng; z += 2) {
-        group(z, std::false_type{}, std::true_type{});
-        if (z + 1 < ng) group(z + 1, std::false_type{}, std::false_type{});
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Decode pass 2 over every group of a KV head in one workgroup that walks a
-// run of keys in 256-key chunks (up to kDecodeLoopMaxSub groups of at most 16
-// columns: a few rows over a long cache, one round of (nwg_pv, kv_heads)
-// workgroups). First the exact maxima of every group's columns (two groups'
-// pass-1 maxima in flight). Then per chunk: the V tiles staged in LDS once for
-// all the groups; for each group in turn the exponentials (hi + lo P columns
-// in LDS, the column sums added up per wave in LDS), the next group's scores
-// requested, and P.V into the group's accumulator (the hi and the lo block
-// into one), which stays in registers over the whole run, the V^T operands
-// read from LDS for each group in parts of two tiles; the next chunk's V
-// tiles are requested after the last group (held in registers during the
-// groups, they spilled). The partials and column sums go where decode_pv
-// puts them, so the combine is the same. Each column carries its row's
+// Decode pass 2 over every group of a KV head in one workgroup (up to NG
+// groups of at most 16 columns: a few rows, or one row of more than 16 query
+// heads), a run of whole tiles each, in chunks of TC tiles. Grid (nwg_pv,
+// kv_heads), 512 threads. Per chunk:
+//   exponentials  two waves take a tile's, half of the groups each (one group:
+//                 half of each lane's keys), in the layout of the P.V MFMA's B operand (lane (j, G): keys
+//                 8G .. 8G+7 of column j), straight from the scores: eight
+//                 consecutive floats per lane
+//   V             the same waves store the tile
+//   P.V           wave w takes the dimensions [D/8 w, D/8 (w + 1)) over all
+//                 tiles, hi and lo into one accumulator per group
+// The chunk's V and P meet in LDS between two barriers; the next chunk's
+// exponentials stand between this one's MFMAs, its V tiles are requested before
+// them and the scores of the chunk after next behind them, so that the stream,
+// the matrix cores and the VALU run at once. A workgroup's run is whole tiles,
+// so that a cache just past one round of workgroups costs each a tile more.
+// Bound by its phases' latency over short runs and by the stream over long
+// ones. Before (a group at a time, its P columns through LDS element by
+// element, two barriers each): 21.8 us of a call for 8 rows of 8 heads on 2 KV
+// heads after 32 760 keys and 36.5 after 32 768, now 14.4 and 16.1; whole calls
+// at decode_pv_groups_ok.
+// The partials go where decode_pv puts them. Each column carries its row's
 // causal limit.
 // ---------------------------------------------------------------------------
-template <int D>
-__global__ __launch_bounds__(512, 1) void decode_pv_all_loop(DecodeArgs a)
+template <int D, int NG>
+__global__ __launch_bounds__(512, 1) void decode_pv_groups(DecodeArgs a)
 {
-    constexpr int W = 8, NCB = 2, THREADS = 64 * W, KEYS = W * kKeyTile, PS = KEYS + 8;
-    constexpr int DB = D / 16, DBW = DB / W, nh = 8 * NCB, HC = nh / 2, MS = kDecodeLoopMaxSub;
-    static_assert(DB % W == 0, "each wave takes whole dimension blocks");
-    static_assert(MS * W * kDecodeMaxGroup <= THREADS, "one thread per column sum to clear");
-    constexpr int T = THREADS / nh, BATCH = 8;                  // lanes per column's maxima
-    __shared__ __attribute__((aligned(16))) uint16_t vt[W][kKeyTile * D];
-    __shared__ __attribute__((aligned(16))) uint16_t pc[2 * kDecodeMaxGroup * PS];
-    __shared__ float smax[MS][kDecodeMaxGroup];
-    __shared__ float lsum[MS][W][kDecodeMaxGroup];
-    __shared__ int crow[MS][kDecodeMaxGroup];                   // the row of group z's column h
-    const int wg = static_cast<int>(blockIdx.x), tid = threadIdx.x;
-    const int kvh0 = static_cast<int>(blockIdx.y) * a.sub, ng = a.sub;     // 2 <= ng <= MS
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, j = l & 15, G = l >> 4;
+    constexpr int TC = 4, CK = TC * kKeyTile;                   // tiles and keys per chunk
+    constexpr int NE = NG > 1 ? NG / 2 : 1;                     // groups whose exponentials a wave takes
+    constexpr int KE = NG > 1 ? 8 : 4;                          // of them each lane's keys
+    constexpr int DB = D / 128;                                 // 16-dimension blocks per wave
+    constexpr int VL = kKeyTile * (D / 8) / 128;                // 16-byte chunks of V per lane
+    constexpr int V_U16 = TC * kKeyTile * D, P_U16 = TC * NG * 2 * 512;
+    constexpr int T = 512 / (16 * NG), BATCH = NG < 4 ? 4 * NG : 16;    // lanes per column's maxima
+    static_assert(D % 128 == 0 && T >= 4 && T <= 32, "whole blocks per wave, whole lane groups per column");
+    __shared__ __attribute__((aligned(16))) uint16_t lds[V_U16 + P_U16];
+    __shared__ float smax[NG][16];
+    __shared__ float lred[NG][NG > 1 ? TC : 8][16];             // by tile, or tile and half
+    uint16_t *vt = lds, *pb = lds + V_U16;
+    const int tid = threadIdx.x, l = tid & 63, j = l & 15, G = l >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wt = wave >> 1, wh = wave & 1;                    // exponentials and V: tile, half of it
+    const int wg = static_cast<int>(blockIdx.x), ng = a.sub, kvh0 = static_cast<int>(blockIdx.y) * ng;
     const uint64_t j0 = static_cast<uint64_t>(wg) * static_cast<uint64_t>(a.keys_pv);
     const uint64_t j1 = j0 + static_cast<uint64_t>(a.keys_pv) < a.n ? j0 + static_cast<uint64_t>(a.keys_pv) : a.n;
     const uint16_t *vbase = a.v + static_cast<uint64_t>(blockIdx.y) * a.kv_stride;
-    const int key_e = tid % KEYS;
-    const int hq = __builtin_amdgcn_readfirstlane(tid / KEYS);  // the same in a whole wave
-    const int jh = tid / T, u = tid % T;
-    // group z's scores of this thread's key of the chunk at c0 (columns hq + 2 i),
-    // in buffer z % 2, requested one group ahead
-    float sva[HC], svb[HC];
-    auto load_scores = [&](int z, uint64_t c0, float(&sv)[HC]) {
-        const uint64_t gk = c0 + key_e, key = gk < j1 ? gk : 0;
-        const int kvh = kvh0 + z;
+    const int zb = NG > 1 ? NE * wh : 0, kb = NG > 1 ? 0 : KE * wh;  // this wave's first group, each lane's first key
+
+    f32x4 sc[NE][KE / 4];
+    auto load_scores = [&](uint64_t c0) {
+        const uint64_t t0 = c0 + static_cast<uint64_t>(kKeyTile * wt);
+        const uint64_t k0 = (t0 < j1 ? t0 : 0) + static_cast<uint64_t>(8 * G + kb);  // (a tile's end stays below npad)
 #pragma unroll
-        for (int i = 0; i < HC; i++) {
-            const int h = hq + 2 * i;
-            const float *col = a.scores + static_cast<uint64_t>(kvh * a.g + (h < a.g ? h : 0)) * a.npad;
-            sv[i] = col[key];
+        for (int i = 0; i < NE; i++) {
+            const int z = zb + i < ng ? zb + i : 0;
+            const float *col = a.scores + static_cast<uint64_t>((kvh0 + z) * a.g + (j < a.g ? j : 0)) * a.npad + k0;
+#pragma unroll
+            for (int k = 0; k < KE / 4; k++) sc[i][k] = *reinterpret_cast<const f32x4 *>(col + 4 * k);
         }
     };
-    // group z's first batch of pass-1 maxima, in buffer z % 2 (two groups' in
-    // flight)
-    auto load_max = [&](int z, float(&mx)[BATCH]) {
-        const float *msrc = a.wgmax + (static_cast<uint64_t>(kvh0 + z) * a.g + (jh < a.g ? jh : 0)) * a.nwg_qk;
+    u32x4 vr[VL];
+    auto tile_keys = [&](uint64_t c0) {                         // valid keys of this wave's tile
+        const uint64_t t0 = c0 + static_cast<uint64_t>(kKeyTile * wt);
+        return t0 < j1 ? static_cast<int>(j1 - t0 < kKeyTile ? j1 - t0 : kKeyTile) : 0;
+    };
+    auto load_v = [&](uint64_t c0) {
+        const int nv = tile_keys(c0);
+        const uint16_t *tb = vbase + (nv ? c0 + static_cast<uint64_t>(kKeyTile * wt) : 0) * D;
 #pragma unroll
-        for (int b = 0; b < BATCH; b++) {
-            const int w = u + b * T;
-            mx[b] = msrc[w < a.nwg_qk ? w : 0];
+        for (int i = 0; i < VL; i++) {
+            const int c = 64 * VL * wh + l + 64 * i, key = c / (D / 8), dc = c % (D / 8);
+            const uint32_t off = key < nv ? static_cast<uint32_t>(key * D + 8 * dc) : 0u;
+            vr[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(tb + off));
         }
     };
-    // the first two groups' maxima, the first chunk's scores of group 0 and
-    // its V tiles
-    float mxa[BATCH], mxb[BATCH];
-    load_max(0, mxa);
-    load_max(1, mxb);
-    load_scores(0, j0, sva);
-    u32x4 vr[Tile<D, 64>::kPer];
-    tile_gload<D, 64, true>(vbase, j0 + kKeyTile * wave, j1, l, vr);
-    __builtin_amdgcn_sched_barrier(0);                          // all loads issued first
-    // the exact maxima, group by group (the sink joins them)
+    auto store_v = [&](uint64_t c0) {
+        const int nv = tile_keys(c0);
+        uint16_t *st = vt + wt * kKeyTile * D;
 #pragma unroll
-    for (int z = 0; z < MS; z++) {
-        if (z < ng) {
-            float(&mx)[BATCH] = (z & 1) ? mxb : mxa;
-            float m = kNegInf;
-#pragma unroll
-            for (int b = 0; b < BATCH; b++) m = (u + b * T < a.nwg_qk && mx[b] > m) ? mx[b] : m;
-            if (z + 2 < ng) load_max(z + 2, mx);
-            const float *msrc = a.wgmax + (static_cast<uint64_t>(kvh0 + z) * a.g + (jh < a.g ? jh : 0)) * a.nwg_qk;
-            for (int w0 = u + BATCH * T; w0 < a.nwg_qk; w0 += BATCH * T) {
-                float xb[BATCH];
-#pragma unroll
-                for (int b = 0; b < BATCH; b++) {
-                    const int w = w0 + b * T;
-                    xb[b] = msrc[w < a.nwg_qk ? w : 0];
-                }
-#pragma unroll
-                for (int b = 0; b < BATCH; b++) m = (w0 + b * T < a.nwg_qk && xb[b] > m) ? xb[b] : m;
-            }
-            m = group_max_hi(m, T);
-            if (a.sink_on) m = m > a.sink ? m : a.sink;
-            if (u == T - 1 && jh < a.g) smax[z][jh] = m;
+        for (int i = 0; i < VL; i++) {
+            const int c = 64 * VL * wh + l + 64 * i, key = c / (D / 8), dc = c % (D / 8);
+            store16(st + key * D + 8 * swz16<D>(key, dc), key < nv ? vr[i] : u32x4{0, 0, 0, 0});
         }
-    }
-    if (tid < MS * W * kDecodeMaxGroup) (&lsum[0][0][0])[tid] = 0.0f;
-    if (tid < MS * kDecodeMaxGroup) (&crow[0][0])[tid] = ((tid / kDecodeMaxGroup) * a.g + tid % kDecodeMaxGroup) / a.G;
-    f32x4 o[MS][DBW] = {};                                      // hi and lo P blocks into one accumulator
-    for (uint64_t c0 = j0; c0 < j1; c0 += KEYS) {
-        const uint64_t c1 = c0 + KEYS < j1 ? c0 + KEYS : j1;
-        const uint64_t gk = c0 + key_e;
-        const bool kv_e = gk < c1, more = c1 < j1;
-        // every wave's P.V of the previous chunk has read the V tiles (first:
-        // the maxima and the cleared sums are visible)
-        __syncthreads();
-        tile_mask_lstore_v16<D, 64>(vt[wave], c0 + kKeyTile * wave, c1, l, vr);
-        auto group = [&](auto zt) {
-            constexpr int z = decltype(zt)::value;
-            float(&sv)[HC] = (z & 1) ? svb : sva;
-            // column h's row sees keys [0, past + row]: key c0 + key_e while
-            // key_e <= past + row - c0, a limit in [-1, KEYS] in a scalar
-            // register; the rows are read from LDS in the chunk loop (held
-            // in registers for every group and column over the loop, they
-            // spilled)
-            float ev[HC];
-            const int64_t rel0 = static_cast<int64_t>(a.past) - static_cast<int64_t>(c0);
+    };
+
+    // the columns' maxima over pass 1's workgroups, T lanes each; the first
+    // chunk's loads behind the first batch of them
+    {
+        const int cz = tid / (16 * T), ch = tid / T % 16, u = tid % T;
+        const float *msrc =
+            a.wgmax + (static_cast<uint64_t>(kvh0 + (cz < ng ? cz : 0)) * a.g + (ch < a.g ? ch : 0)) * a.nwg_qk;
+        float mx[BATCH];
+        auto load_max = [&](int w0) {                           // (past the last: the first again)
 #pragma unroll
-            for (int i = 0; i < HC; i++) {
-                const int h = hq + 2 * i;
-                const int64_t rel = rel0 + __builtin_amdgcn_readfirstlane(crow[z][h]);
-                const int lim = __builtin_amdgcn_readfirstlane(static_cast<int>(rel < 0 ? -1 : rel > KEYS ? KEYS : rel));
-                const bool vis = (h < a.g) & kv_e & (key_e <= lim);
-                const float x = exp_poly(sv[i] - smax[z][h]);   // computed in every lane, then selected
-                ev[i] = vis ? x : 0.0f;
-            }
-            // the next group's scores, or the next chunk's of group 0 (this
-            // buffer's scores are used above)
-            if (z + 1 < ng) load_scores(z + 1, c0, ((z + 1) & 1) ? svb : sva);
-            else if (more) load_scores(0, c1, sva);
-#pragma unroll
-            for (int i = 0; i < HC; i += 2) {
-                const int h = hq + 2 * i;                       // slots i and i + 1: columns h, h + 2
-                uint32_t hb, lb;
-                split2(ev[i], ev[i + 1], hb, lb);
-                pc[h * PS + key_e] = static_cast<uint16_t>(hb);
-                pc[(h + 2) * PS + key_e] = static_cast<uint16_t>(hb >> 16);
-                pc[(nh + h) * PS + key_e] = static_cast<uint16_t>(lb);
-                pc[(nh + h + 2) * PS + key_e] = static_cast<uint16_t>(lb >> 16);
-            }
-            float esum[HC];
-#pragma unroll
-            for (int i = 0; i < HC; i++) esum[i] = wave_sum_hi(ev[i]);
-            if (l == 63) {
-#pragma unroll
-                for (int i = 0; i < HC; i++) lsum[z][wave][hq + 2 * i] += esum[i];
-            }
-            __syncthreads();                                    // the P columns (and V tiles) are in LDS
-            // P.V in parts of TP tiles, each part's P and V^T operands read
-            // from LDS before its MFMAs; the last part's are read before the
-            // barrier after which pc is written again
-            constexpr int TP = 2;
-            auto part = [&](auto pt) {
-                constexpr int t0 = decltype(pt)::value * TP;
-                constexpr bool LAST = t0 + TP == W;
-                u32x4 bp[TP][NCB], av[TP][DBW];
-#pragma unroll
-                for (int t = 0; t < TP; t++) {
-#pragma unroll
-                    for (int c = 0; c < NCB; c++) bp[t][c] = load16(pc + (16 * c + j) * PS + kKeyTile * (t0 + t) + 8 * G);
-#pragma unroll
-                    for (int db = 0; db < DBW; db++) av[t][db] = vt16_operand<D>(vt[t0 + t], 16 * (wave * DBW + db), l);
-                }
-                if constexpr (LAST) __syncthreads();
-#pragma unroll
-                for (int t = 0; t < TP; t++)
-#pragma unroll
-                    for (int db = 0; db < DBW; db++)
-#pragma unroll
-                        for (int c = 0; c < NCB; c++) o[z][db] = mfma16(av[t][db], bp[t][c], o[z][db]);
-                __builtin_amdgcn_sched_barrier(0);
-            };
-            part(std::integral_constant<int, 0>{});
-            part(std::integral_constant<int, 1>{});
-            part(std::integral_constant<int, 2>{});
-            part(std::integral_constant<int, 3>{});
+            for (int b = 0; b < BATCH; b++) mx[b] = msrc[w0 + b * T < a.nwg_qk ? w0 + b * T : 0];
         };
-        group(std::integral_constant<int, 0>{});
-        group(std::integral_constant<int, 1>{});
-        if constexpr (MS > 2) { if (ng > 2) group(std::integral_constant<int, 2>{}); }
-        if constexpr (MS > 3) { if (ng > 3) group(std::integral_constant<int, 3>{}); }
-        // the next chunk's V tiles (requested here, where the P.V operands
-        // are no longer held)
-        if (more) tile_gload<D, 64, true>(vbase, c1 + kKeyTile * wave, j1, l, vr);
+        load_max(u);
+        load_scores(j0);
+        load_v(j0);
+        __builtin_amdgcn_sched_barrier(0);                      // all loads issued first
+        float m = kNegInf;
+#pragma unroll
+        for (int b = 0; b < BATCH; b++) m = fmaxnn(m, mx[b]);
+        for (int w0 = u + BATCH * T; w0 < a.nwg_qk; w0 += BATCH * T) {
+            load_max(w0);
+#pragma unroll
+            for (int b = 0; b < BATCH; b++) m = fmaxnn(m, mx[b]);
+        }
+        m = fmaxnn(m, dpp<0xB1, 0xF>(m, kNegInf));
+        m = fmaxnn(m, dpp<0x4E, 0xF>(m, kNegInf));
+        if (T >= 8) m = fmaxnn(m, dpp<0x141, 0xF>(m, kNegInf));
+        if (T >= 16) m = fmaxnn(m, dpp<0x140, 0xF>(m, kNegInf));
+        if (T >= 32) m = fmaxnn(m, dpp<0x142, 0xA>(m, kNegInf));
+        if (a.sink_on) m = m > a.sink ? m : a.sink;             // the sink joins the maximum
+        if (u == T - 1) smax[cz][ch] = m;
     }
-    __syncthreads();                                            // the column sums are complete
+    lds_barrier();
+    // this lane's columns: exponential, last visible key (from j0; a run is at
+    // most 2^30 keys)
+    float ec[NE], eb[NE], lsum[NE];
+    int lim[NE];
 #pragma unroll
-    for (int z = 0; z < MS; z++) {
-        if (z < ng) {
-            const uint64_t pbase = (static_cast<uint64_t>(kvh0 + z) * a.nwg_pv + wg) * a.g;
+    for (int i = 0; i < NE; i++) {
+        const RowExp x(smax[zb + i][j]);
+        ec[i] = x.c;
+        eb[i] = x.b;
+        lsum[i] = 0.0f;
+        const int64_t last = static_cast<int64_t>(a.past) + ((zb + i) * a.g + j) / a.G - static_cast<int64_t>(j0);
+        lim[i] = static_cast<int>(last < -1 ? -1 : last > (1 << 30) ? 1 << 30 : last);
+    }
+    // exponential e of the chunk at c0 (of this wave's KE NE): key kb + e % KE of
+    // column (zb + e / KE, j); none is visible where the chunk is not there
+    uint32_t ph[NE][KE / 2], pl[NE][KE / 2];
+    float ev[2];
+    auto exp_one = [&](int e, uint64_t c0, bool there) {
+        const int i = e / KE, k = e % KE;
+        // keys 0 .. vis of the lane's
+        const int vis = there ? lim[i] - (static_cast<int>(c0 - j0) + kKeyTile * wt + 8 * G + kb) : -1;
+        RowExp x(0.0f);
+        x.c = ec[i];
+        x.b = eb[i];
+        const float y = exp_score(sc[i][k / 4][k % 4], x);
+        ev[k & 1] = k <= vis ? y : 0.0f;
+        lsum[i] += ev[k & 1];
+        if (k & 1) split2(ev[0], ev[1], ph[i][k >> 1], pl[i][k >> 1]);
+    };
 #pragma unroll
-            for (int db = 0; db < DBW; db++) {
-                if (j < a.g) {
-                    float *dst = a.part_o + (pbase + j) * D + 16 * (wave * DBW + db) + 4 * G;
-                    *reinterpret_cast<float4 *>(dst) = float4{o[z][db][0], o[z][db][1], o[z][db][2], o[z][db][3]};
+    for (int e = 0; e < KE * NE; e++) exp_one(e, j0, wt * kKeyTile < static_cast<int>(j1 - j0));
+    if (j0 + CK < j1) load_scores(j0 + CK);
+    f32x4 o[NG][DB] = {};
+    for (uint64_t c0 = j0; c0 < j1; c0 += CK) {
+        const int nt = static_cast<int>((j1 - c0 < CK ? j1 - c0 + kKeyTile - 1 : CK) / kKeyTile);
+        lds_barrier();                                          // the last chunk's operands are read
+        store_v(c0);
+#pragma unroll
+        for (int i = 0; i < NE; i++) {
+            uint16_t *dst = pb + (wt * NG + zb + i) * 2 * 512 + 8 * l + kb;
+            if constexpr (KE == 8) {
+                store16(dst, u32x4{ph[i][0], ph[i][1], ph[i][2], ph[i][3]});
+                store16(dst + 512, u32x4{pl[i][0], pl[i][1], pl[i][2], pl[i][3]});
+            } else {
+                *reinterpret_cast<u32x2 *>(dst) = u32x2{ph[i][0], ph[i][1]};
+                *reinterpret_cast<u32x2 *>(dst + 512) = u32x2{pl[i][0], pl[i][1]};
+            }
+        }
+        const uint64_t cn = c0 + CK;
+        if (cn < j1) load_v(cn);
+        __builtin_amdgcn_sched_barrier(0);
+        lds_barrier();                                          // the chunk's V and P are in LDS
+        // this wave's tile of the next chunk holds keys
+        const bool there = cn + static_cast<uint64_t>(kKeyTile * wt) < j1;
+#pragma unroll
+        for (int t = 0; t < TC; t++) {
+            if (t < nt) {
+                u32x4 av[DB];
+#pragma unroll
+                for (int db = 0; db < DB; db++) av[db] = vt16_operand<D>(vt + t * kKeyTile * D, 16 * (wave * DB + db), l);
+                constexpr int ZP = NG < 4 ? NG : 4;              // groups whose P operands are held
+#pragma unroll
+                for (int z0 = 0; z0 < NG; z0 += ZP) {
+                    u32x4 bp[ZP][2];
+#pragma unroll
+                    for (int z = 0; z < ZP; z++)
+#pragma unroll
+                        for (int c = 0; c < 2; c++) bp[z][c] = load16(pb + ((t * NG + z0 + z) * 2 + c) * 512 + 8 * l);
+                    __builtin_amdgcn_sched_barrier(0);
+                    // the next chunk's exponentials dealt out over the MFMAs
+                    // (groups past ng: their P is another's, never stored)
+                    constexpr int M = 2 * ZP * DB, EP = KE * NE / TC * ZP / NG;     // MFMAs, exponentials
+#pragma unroll
+                    for (int m = 0; m < M; m++) {
+                        const int c = m / (ZP * DB), z = m / DB % ZP, db = m % DB;
+                        o[z0 + z][db] = mfma16(av[db], bp[z][c], o[z0 + z][db]);
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int e = EP * m / M; e < EP * (m + 1) / M; e++)
+                            exp_one(KE * NE / TC * t + EP * (z0 / ZP) + e, cn, there);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
                 }
             }
-            if (tid < a.g) {
-                // columns of parity p were summed by waves 4 p .. 4 p + 3
-                const int p0 = (tid % (THREADS / KEYS)) * (KEYS / 64);
-                float L = 0.0f;
-                for (int w = 0; w < KEYS / 64; w++) L += lsum[z][p0 + w][tid];
-                if (a.sink_on && wg == 0) L += exp_poly(a.sink - smax[z][tid]);  // once per column
-                a.part_l[pbase + tid] = L;
-            }
+        }
+        if (cn + CK < j1) load_scores(cn + CK);
+    }
+    // the column sums: over the lanes of a column, then the tiles' waves
+#pragma unroll
+    for (int i = 0; i < NE; i++) {
+        lsum[i] += __shfl_xor(lsum[i], 16);
+        lsum[i] += __shfl_xor(lsum[i], 32);
+        if (G == 0) lred[zb + i][NG > 1 ? wt : wave][j] = lsum[i];
+    }
+    if (j < a.g) {
+        const uint64_t zs = static_cast<uint64_t>(a.nwg_pv) * a.g;       // cells of a group
+        float *dst = a.part_o + (kvh0 * zs + static_cast<uint64_t>(wg) * a.g + j) * D + 16 * DB * wave + 4 * G;
+#pragma unroll
+        for (int z = 0; z < NG; z++, dst += zs * D)
+            if (z < ng)
+#pragma unroll
+                for (int db = 0; db < DB; db++) *reinterpret_cast<f32x4 *>(dst + 16 * db) = o[z][db];
+    }
+    lds_barrier();
+    if (tid < 16 * NG) {
+        const int z = tid / 16, h = tid % 16;
+        if (z < ng && h < a.g) {
+            float L = 0.0f;
+#pragma unroll
+            for (int t = 0; t < (NG > 1 ? TC : 8); t++) L += lred[z][t][h];
+            if (a.sink_on && wg == 0) L += exp_poly(a.sink - smax[z][h]);    // once per column
+            a.part_l[(static_cast<uint64_t>(kvh0 + z) * a.nwg_pv + wg) * a.g + h] = L;
         }
     }
 }
@@ -1918,50 +1819,15 @@ __device__ __forceinline__ u32x4 q_chunk(u32x4 v, bool valid, uint32_t sign)
     return valid ? v ^ sign : u32x4{0, 0, 0, 0};
 }
 
-// One row's exponential: see exp_score.
-struct RowExp {
-    float c, b;
-    // m: the row's maximum dot product; with the sink, ms receives the scaled
-    // maximum, the larger of the scores' and the sink (vmaxss,
-    // decode.rs:239-290). Where the exponent of the maximum itself would leave
-    // the f32 range, two scores that differ at all differ by far more than the
-    // exponential's clamp, and a smaller c tells them apart as well.
-    __device__ __forceinline__ RowExp(const PrefillArgs &a, float m, bool sink, float &ms)
-    {
-        const float s = __builtin_fabsf(a.scale);
-        c = s * 1.442695f;
-        const float sm = m * s;
-        const bool over = sink && !(sm > a.sink);
-        ms = over ? a.sink : sm;
-        float t = over ? a.sink * 1.442695f : m * c;
-        if (__builtin_fabsf(t) > 1e38f) {
-            c *= 0x1p-24f;
-            t = over ? a.sink * (1.442695f * 0x1p-24f) : m * c;
-        }
-        b = 0.5f - t;
-    }
-};
-
-// P(x - M) of the score x whose dot product is acc: t = (x - M) log2(e) + 1/2
-// in one rounding, clamped as the emitted exponential clamps (a NaN too), k =
-// floor(t), and the emitted polynomial about t - k - 1/2, its argument moved
-// by 1/2 into the coefficients: P(x) 2^k = Q(t - k) 2^k. Nine instructions
-// where subtract, clamp, scale, round, subtract, convert, polynomial and
-// ldexp take eleven (and one more for a scale that is no power of two): the
-// causal passes are VALU-bound up to D = 128. Against 64-bit exponentials over
-// |score - M| up to 30, relative rms 1.42e-5 and largest 6.1e-5, both the
-// polynomial's own and the same either way.
-__device__ __forceinline__ float exp_score(float acc, const RowExp &x)
+// A causal row's exponential: m its maximum dot product; with the sink, ms
+// receives the scaled maximum, the larger of the scores' and the sink (vmaxss,
+// decode.rs:239-290).
+__device__ __forceinline__ RowExp causal_exp(const PrefillArgs &a, float m, bool sink, float &ms)
 {
-    const float t = __builtin_fmaxf(__builtin_fmaf(acc, x.c, x.b), -125.49977f);
-    int k;
-    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(k) : "v"(t));
-    const float f = __builtin_amdgcn_fractf(t);
-    float p = __builtin_fmaf(f, 0.00967248f, 0.03615915f);
-    p = __builtin_fmaf(f, p, 0.17147906f);
-    p = __builtin_fmaf(f, p, 0.4897125f);
-    p = __builtin_fmaf(f, p, 0.70714957f);
-    return __builtin_ldexpf(p, k);
+    const float s = __builtin_fabsf(a.scale), c = s * 1.442695f, sm = m * s;
+    const bool over = sink && !(sm > a.sink);
+    ms = over ? a.sink : sm;
+    return RowExp(c, over ? a.sink : m, over ? 1.442695f : c);
 }
 
 // A row's normalisation: the division by its sum, or (the sink) the
@@ -2158,7 +2024,7 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_attn(PrefillArgs a)
     }
     m = __builtin_fmaxf(m, __shfl_xor(m, 32));
     float ms;                                                   // the scaled maximum, with the sink
-    const RowExp ex(a, m, SINK, ms);
+    const RowExp ex = causal_exp(a, m, SINK, ms);
 
     // pass 2: exponentials at the exact maximum, P.V with P = hi + lo
     f32x16 o[D / 32];
@@ -2295,7 +2161,7 @@ __global__ __launch_bounds__(64 * KS, 1) void prefill_ks(PrefillArgs a)
     // rows past the chunk: a finite maximum, their outputs are never stored
     if (!rowv) m = 0.0f;
     float ms;
-    const RowExp ex(a, m, false, ms);
+    const RowExp ex = causal_exp(a, m, false, ms);
 
     // pass 2: exponentials of the kept scores at the exact maximum, P.V with
     // P = hi + lo
@@ -2576,7 +2442,7 @@ __global__ __launch_bounds__(64 * KS, 1) void prefill_kd(PrefillArgs a)
     // rows past the chunk: a finite maximum, their outputs are never stored
     if (!rowv) m = 0.0f;
     float ms;
-    const RowExp ex(a, m, false, ms);
+    const RowExp ex = causal_exp(a, m, false, ms);
 
     // pass 2. exps_q(r, q): the exponentials of scores 4q .. 4q+3 of this
     // wave's tile of round r at the exact maximum, masked by bits (so that the
@@ -2902,7 +2768,7 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_split_pv(PrefillArgs a, Sp
                 m = __builtin_fmaxf(m, sp.smax[(static_cast<uint64_t>(z) * sp.heads + head) * a.rows + row]);
         }
         float ms;                                                   // the scaled maximum, with the sink
-        const RowExp ex(a, m, SINK, ms);
+        const RowExp ex = causal_exp(a, m, SINK, ms);
 
         u32x4 qb[D / 16];
         const uint16_t *qp = a.q + (rowv ? row : 0) * a.q_row + static_cast<uint64_t>(head) * a.q_head;

@@ -55,7 +55,7 @@ struct DecodeArgs {
     // y G + c % G, whose visible keys are [0, past + row].
     int xcd;                // 1: the groups of a key range numbered onto one XCD (several groups)
     int qk_all;             // 1: pass 1 scores all sub groups of a KV head in each workgroup
-    int pv_all;             // 1: pass 2 (256-key workgroups) takes all sub groups in each workgroup
+    int pv_all;             // 1: pass 2 takes all sub groups in each workgroup (decode_pv_groups)
     int direct;             // 1: pass 2 writes the outputs itself (decode_direct_ok), no combine
     int rows;               // 1 for a decode step
     int G;                  // query heads per KV head
@@ -206,9 +206,6 @@ constexpr int kDecodeMaxRows = 16;
 constexpr int kDecodeMaxCols = 8 * kDecodeMaxGroup;     // columns per KV head
 // pass 1 scores up to this many groups of a KV head in one workgroup
 constexpr int kDecodeMaxSub = 8;
-// pass 2 walks a run of keys for up to this many groups of a KV head in one
-// workgroup (their accumulators stay in registers over the run)
-constexpr int kDecodeLoopMaxSub = 4;
 // Past 8 rows or 64 columns (up to 16 rows, 128 columns) the few-rows decode
 // beats the split causal kernel only while its groups times the visible keys
 // stay small: 16/2 heads at D = 256, 9 and 16 rows after 32K 110 -> 49 and 114
@@ -259,35 +256,35 @@ inline bool decode_direct_ok(int d, int rows, int sub, int g, uint64_t n, bool f
 // Pass 2 in chunks (one round of workgroups over a long cache) is built for
 // the tuned head dimensions; under the Fused form at D = 256 for one row in
 // groups of up to 8 columns (with 16 its running maxima and corrections and
-// the P columns' operands no longer fit beside the next chunk's V tile).
+// the P columns' operands no longer fit beside the next chunk's V tile), under
+// the Chained form where decode_pv_groups does not take the call.
 inline bool decode_pv_loop_ok(int d, int g, int rows, bool fused)
 {
     return d == 64 || d == 128 || (d == 256 && (!fused || (g <= 8 && rows == 1)));
 }
-// Several rows at D = 256 in 2 or more groups: pass 2 over all the groups of
-// a KV head per workgroup loads each V tile once for all of them; chunked
-// runs per group stream V once per group, but in one round of workgroups.
-// The runs go with at most 4 groups where the all-group form would take more
-// than one round of 256-key workgroups (kv_chunks = kv_heads x ceil(n/256)):
-// 16/2 heads at D = 256, 4 rows after 64K and 128K 58.7 -> 55.3 and 105.6 ->
-// 90.9 us, 8 rows after 128K 147.9 -> 139.8; but 8 rows after 32K (one round)
-// 46.2 -> 49.0 and 16 rows (8 groups) after 64K 126.6 -> 131.4.
-inline bool decode_pv_loop_rows_ok(int d, int rows, int sub, uint64_t kv_chunks, uint64_t cus)
+// Pass 2 over every group of a KV head in one workgroup (decode_pv_groups),
+// past one round of 256-key workgroups per group (below, the groups'
+// exponentials run beside each other on compute units that would idle: 8 rows
+// of 8 heads on 2 KV heads after 1000 and 8184 keys 14.6 and 20.5 us, 17.0 and
+// 23.8 this way). Past it, us a call by a group or a round of 256-key
+// workgroups at a time and this way: 8 rows after 8 192 27.8 -> 26.0, 32 768
+// 57.6 -> 41.0, 131 000 116 -> 90; 4 rows after 32 764 30.9 -> 28.8, 65 536
+// 54 -> 45; 16 rows after 32 752 58.7 -> 54.0; 2 rows (one group of 16
+// columns) after 32 768 29.6 -> 26.5; 32 heads per KV head at 33 000 40 ->
+// 33. One group of at most 8 columns takes it only where the run of tiles
+// leaves the 256-key chunks of decode_pv one or two tiles over (`run` whole
+// tiles a workgroup), which costs those a whole chunk: one row at 32 769 and
+// 40 001 25.4 and 27.0 -> 24.5 and 26.4, but 49 153 and 131 072 (12 and 32
+// tiles) 29.7 and 55.9 -> 31.3 and 58.4. Runs past 2^25 tiles (2^30 keys) are
+// left to decode_pv.
+inline bool decode_pv_groups_dim(int d, int sub) { return d == 256 && sub >= 1 && sub <= kDecodeMaxSub; }
+inline bool decode_pv_groups_ok(int d, int sub, int g, uint64_t run)
 {
-    return d != 256 || rows == 1 || sub == 1 || (sub <= 4 && kv_chunks > cus);
+    const bool rest = run % 8 == 1 || run % 8 == 2;
+    return decode_pv_groups_dim(d, sub) && run <= (uint64_t{1} << 25) && (sub > 1 || g > 8 || (rest && run < 32));
 }
-// Several rows at D = 256 in 3 to kDecodeLoopMaxSub groups where pass 1 takes
-// every group of a KV head in one workgroup and 256-key pass-2 workgroups
-// would take more than one round: one round of workgroups that each walk a
-// run of keys for all the groups (decode_pv_all_loop; each V tile loaded once
-// for all the groups, where a run per group streams V once per group). 8 rows
-// of 8 heads (4 groups) after 64K / 128K: 73.8 / 130.9 -> 70.6 / 120.5 us;
-// with 2 groups the runs per group were as fast (4 rows: 50.6 / 87.5 against
-// 51.6 / 88.7 us).
-inline bool decode_pv_all_loop_ok(int d, int rows, int sub, bool qk_all, uint64_t kv_chunks, uint64_t cus)
-{
-    return d == 256 && rows > 1 && sub >= 3 && sub <= kDecodeLoopMaxSub && qk_all && kv_chunks > cus;
-}
+// Its workgroups per KV head: one round of the compute units.
+inline uint64_t decode_pv_groups_wgs(uint64_t kv_heads, uint64_t cus) { return cus > kv_heads ? cus / kv_heads : 1; }
 hipError_t launch_layer_prep(const LayerPrepArgs &a, hipStream_t s);
 hipError_t launch_norm_rope(const NormRopeArgs &a, hipStream_t s);
 hipError_t launch_gate(const GateArgs &a, hipStream_t s);

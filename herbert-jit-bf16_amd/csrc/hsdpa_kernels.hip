@@ -316,15 +316,14 @@ static hipError_t decode_dm(const DecodeArgs &a, int kv_heads, hipStream_t s)
         }
     }
     if (a.pv_all) {
-        // pass 2 over all the KV head's groups in one workgroup: 256 keys
-        // each, or a run of chunks each (decode_pv_all_loop_ok)
+        // pass 2 over all the KV head's groups in one workgroup
         if constexpr (D == 256) {
-            if (a.keys_pv == kDecodeKeysPV) {
-                e = launch(decode_pv_all<D>, dim3(a.nwg_pv, kv_heads, 1), dim3(512), s, a);
-            } else {
-                if (a.keys_pv < kDecodeKeysPV || a.sub < 2 || a.sub > kDecodeLoopMaxSub) return hipErrorInvalidValue;
-                e = launch(decode_pv_all_loop<D>, dim3(a.nwg_pv, kv_heads, 1), dim3(512), s, a);
-            }
+            const dim3 gall(a.nwg_pv, kv_heads, 1);
+            e = a.sub == 1   ? launch(decode_pv_groups<D, 1>, gall, dim3(512), s, a)
+                : a.sub == 2 ? launch(decode_pv_groups<D, 2>, gall, dim3(512), s, a)
+                : a.sub <= 4 ? launch(decode_pv_groups<D, 4>, gall, dim3(512), s, a)
+                : a.sub <= 8 ? launch(decode_pv_groups<D, 8>, gall, dim3(512), s, a)
+                             : hipErrorInvalidValue;
         } else {
             return hipErrorInvalidValue;
         }
