@@ -2814,19 +2814,28 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_split_pv(PrefillArgs a, Sp
     }
 }
 
-// grid (rows with partials, heads), D threads: one output element each.
-template <int D>
-__global__ __launch_bounds__(D) void prefill_split_combine(PrefillArgs a, SplitArgs sp, int splits);
-// The wide combine's shape: DL lanes of 4 dimensions each, SUBS subsets of
-// the splits; it takes more than kCombineNarrowSplits splits (2 splits of the
-// paired form: 21.0 us with a thread per dimension, 35.6 us this way).
+// The combines' shapes: DL lanes of 4 dimensions a (row, head) cell. Up to
+// kCombineNarrowSplits splits, CELLS cells a workgroup, each lane its splits in
+// turn; beyond, one cell a workgroup, SUBS subsets of the splits (128 splits of
+// 17 rows after 32K keys: 36.6 us with each lane its splits in turn, 8.3 so).
 template <int D> struct CombineShape {
     static constexpr int DL = D / 4, SUBS = 256 / DL > 0 ? 256 / DL : 1, THREADS = DL * SUBS;
+    static constexpr int CELLS = SUBS;
 };
 constexpr int kCombineNarrowSplits = 4;
 template <int D>
+__global__ __launch_bounds__(CombineShape<D>::THREADS) void prefill_split_combine(PrefillArgs a, SplitArgs sp,
+                                                                                  int splits);
+template <int D>
 __global__ __launch_bounds__(CombineShape<D>::THREADS) void prefill_split_combine_wide(PrefillArgs a, SplitArgs sp,
                                                                                        int splits);
+
+// The narrow combine's grid: sp.srows x heads cells.
+template <int D> static dim3 combine_grid(const SplitArgs &sp)
+{
+    const uint64_t cells = sp.srows * static_cast<uint64_t>(sp.heads);
+    return dim3(static_cast<unsigned>((cells + CombineShape<D>::CELLS - 1) / CombineShape<D>::CELLS));
+}
 
 // The three split kernels on grid (row groups, head groups, splits).
 template <int D, int HPW, int NW, bool SINK = false>
@@ -2838,10 +2847,10 @@ static hipError_t launch_prefill_split(const PrefillArgs &a, int heads, const Pr
     hipError_t e = launch(prefill_split_max<D, HPW, NW>, gs, dim3(64 * NW), s, a, sp);
     if (e == hipSuccess) e = launch(prefill_split_pv<D, HPW, NW, false, SINK>, gs, dim3(64 * NW), s, a, sp);
     if (e != hipSuccess) return e;
-    const dim3 gc(static_cast<unsigned>(a.rows), heads);
+    const dim3 block(CombineShape<D>::THREADS);
     return splits > kCombineNarrowSplits
-               ? launch(prefill_split_combine_wide<D>, gc, dim3(CombineShape<D>::THREADS), s, a, sp, splits)
-               : launch(prefill_split_combine<D>, gc, dim3(D), s, a, sp, splits);
+               ? launch(prefill_split_combine_wide<D>, dim3(static_cast<unsigned>(a.rows), heads), block, s, a, sp, splits)
+               : launch(prefill_split_combine<D>, combine_grid<D>(sp), block, s, a, sp, splits);
 }
 
 // The paired form on the causal kernel's grid (row groups, head groups); pr
@@ -2859,23 +2868,68 @@ static hipError_t launch_prefill_paired(const PrefillArgs &a, int heads, const P
     hipError_t e = launch(prefill_split_max<D, HPW, NW>, gmax, dim3(64 * NW), s, a, sp);
     if (e == hipSuccess) e = launch(prefill_split_pv<D, HPW, NW, true, SINK>, grid, dim3(64 * NW), s, a, sp);
     if (e != hipSuccess) return e;
-    return launch(prefill_split_combine<D>, dim3(static_cast<unsigned>(pr.srows), heads), dim3(D), s, a, sp, 2);
+    return launch(prefill_split_combine<D>, combine_grid<D>(sp), dim3(CombineShape<D>::THREADS), s, a, sp, 2);
 }
 
+// One cell's outputs from its sums: 4 dimensions from 4 t on.
 template <int D>
-__global__ __launch_bounds__(D) void prefill_split_combine(PrefillArgs a, SplitArgs sp, int splits)
+__device__ __forceinline__ void combine_store(const PrefillArgs &a, uint64_t row, uint64_t head, int t, f32x4 o, float L)
 {
-    const uint64_t row = sp.r0 + blockIdx.x, head = blockIdx.y;
-    const int dim = threadIdx.x;
-    float o = 0.0f, ls = 0.0f;
-    for (int z = 0; z < splits; z++) {
-        const uint64_t cell = (static_cast<uint64_t>(z) * sp.srows + blockIdx.x) * sp.heads + head;
-        o += sp.so[cell * D + dim];
-        ls += sp.sl[cell];
+    uint16_t ob[4];
+    if (a.sink_on) {
+        const float inv = 1.0f / L;                             // the sink: O times 1 / l
+#pragma unroll
+        for (int r = 0; r < 4; r++) ob[r] = static_cast<uint16_t>(cvt_out(o[r] * inv));
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; r++) ob[r] = static_cast<uint16_t>(cvt_out(o[r] / L));
     }
-    uint16_t ob = static_cast<uint16_t>(cvt_out(a.sink_on ? o * (1.0f / ls) : o / ls));   // the sink: O times 1 / l
-    if (a.gate) ob = gate_bf16(ob, a.gate[row * a.gate_row + head * D + dim]);
-    a.out[row * a.out_row + head * D + dim] = ob;
+    if (a.gate) {
+        const uint2 gw = *reinterpret_cast<const uint2 *>(a.gate + row * a.gate_row + head * D + 4 * t);
+        const uint16_t gv[4] = {static_cast<uint16_t>(gw.x), static_cast<uint16_t>(gw.x >> 16),
+                                static_cast<uint16_t>(gw.y), static_cast<uint16_t>(gw.y >> 16)};
+#pragma unroll
+        for (int r = 0; r < 4; r++) ob[r] = gate_bf16(ob[r], gv[r]);
+    }
+    *reinterpret_cast<uint2 *>(a.out + row * a.out_row + head * D + 4 * t) =
+        uint2{ob[0] | (static_cast<uint32_t>(ob[1]) << 16), ob[2] | (static_cast<uint32_t>(ob[3]) << 16)};
+}
+
+// The combine for up to kCombineNarrowSplits splits: consecutive cells (row,
+// head) of consecutive lanes, so that a slot's partials are read as one
+// contiguous run of 16-byte loads, every split's requested before the sums.
+// Bound by the partials' bytes. Calls with a workgroup of one element a thread
+// for each cell and this way: 1000 rows of 32 heads after 500 at D = 96 77.0 ->
+// 73.2 us, 1000 of 16 after 1000 at D = 256 97.4 -> 93.5, 600 of 16 at D = 96
+// 33.5 -> 31.1.
+template <int D>
+__global__ __launch_bounds__(CombineShape<D>::THREADS) void prefill_split_combine(PrefillArgs a, SplitArgs sp,
+                                                                                  int splits)
+{
+    constexpr int DL = CombineShape<D>::DL, CELLS = CombineShape<D>::CELLS;
+    const int t = static_cast<int>(threadIdx.x) % DL;
+    const uint64_t heads = static_cast<uint64_t>(sp.heads), cells = sp.srows * heads;
+    const uint64_t at = static_cast<uint64_t>(blockIdx.x) * CELLS + threadIdx.x / DL;
+    if (at >= cells) return;
+    f32x4 xo[kCombineNarrowSplits];
+    float xl[kCombineNarrowSplits];
+#pragma unroll
+    for (int z = 0; z < kCombineNarrowSplits; z++)
+        if (z < splits) {
+            const uint64_t cell = static_cast<uint64_t>(z) * cells + at;
+            xo[z] = *reinterpret_cast<const f32x4 *>(sp.so + cell * D + 4 * t);
+            xl[z] = sp.sl[cell];
+        }
+    f32x4 o = xo[0];
+    float L = xl[0];
+#pragma unroll
+    for (int z = 1; z < kCombineNarrowSplits; z++)
+        if (z < splits) {
+            o += xo[z];
+            L += xl[z];
+        }
+    const uint32_t r = static_cast<uint32_t>(at / heads);
+    combine_store<D>(a, sp.r0 + r, at - r * heads, t, o, L);
 }
 
 // The combine for many splits (more than kCombineNarrowSplits).
@@ -2930,25 +2984,7 @@ __global__ __launch_bounds__(CombineShape<D>::THREADS) void prefill_split_combin
         sum.w += x.w;
         L += lred[v];
     }
-    const float sv[4] = {sum.x, sum.y, sum.z, sum.w};
-    uint16_t ob[4];
-    if (a.sink_on) {
-        const float inv = 1.0f / L;                             // the sink: O times 1 / l
-#pragma unroll
-        for (int r = 0; r < 4; r++) ob[r] = static_cast<uint16_t>(cvt_out(sv[r] * inv));
-    } else {
-#pragma unroll
-        for (int r = 0; r < 4; r++) ob[r] = static_cast<uint16_t>(cvt_out(sv[r] / L));
-    }
-    if (a.gate) {
-        const uint2 gw = *reinterpret_cast<const uint2 *>(a.gate + row * a.gate_row + head * D + 4 * t);
-        const uint16_t gv[4] = {static_cast<uint16_t>(gw.x), static_cast<uint16_t>(gw.x >> 16),
-                                static_cast<uint16_t>(gw.y), static_cast<uint16_t>(gw.y >> 16)};
-#pragma unroll
-        for (int r = 0; r < 4; r++) ob[r] = gate_bf16(ob[r], gv[r]);
-    }
-    *reinterpret_cast<uint2 *>(a.out + row * a.out_row + head * D + 4 * t) =
-        uint2{ob[0] | (static_cast<uint32_t>(ob[1]) << 16), ob[2] | (static_cast<uint32_t>(ob[3]) << 16)};
+    combine_store<D>(a, row, head, t, f32x4{sum.x, sum.y, sum.z, sum.w}, L);
 }
 
 }  // namespace hsdpa
