@@ -1216,7 +1216,8 @@ __global__ __launch_bounds__(64 * W, D > 256 ? 1 : 8 / W) void decode_pv(DecodeA
 // heads), a run of whole tiles each, in chunks of TC tiles. Grid (nwg_pv,
 // kv_heads), 512 threads. Per chunk:
 //   exponentials  two waves take a tile's, half of the groups each (one group:
-//                 half of each lane's keys), in the layout of the P.V MFMA's B operand (lane (j, G): keys
+//                 half of each lane's keys; where a chunk has 8 tiles, a wave
+//                 takes a tile's), in the layout of the P.V MFMA's B operand (lane (j, G): keys
 //                 8G .. 8G+7 of column j), straight from the scores: eight
 //                 consecutive floats per lane
 //   V             the same waves store the tile
@@ -1238,26 +1239,31 @@ __global__ __launch_bounds__(64 * W, D > 256 ? 1 : 8 / W) void decode_pv(DecodeA
 template <int D, int NG>
 __global__ __launch_bounds__(512, 1) void decode_pv_groups(DecodeArgs a)
 {
-    constexpr int TC = 4, CK = TC * kKeyTile;                   // tiles and keys per chunk
-    constexpr int NE = NG > 1 ? NG / 2 : 1;                     // groups whose exponentials a wave takes
-    constexpr int KE = NG > 1 ? 8 : 4;                          // of them each lane's keys
+    // tiles per chunk: as many bytes of V either way (with 8 groups at D = 128
+    // the P operands of 8 tiles would not fit beside them)
+    constexpr int TC = D == 128 && NG <= 4 ? 8 : 4, CK = TC * kKeyTile;
+    constexpr int WT = 8 / TC;                                  // waves per tile
+    constexpr bool HALF = NG < WT;                              // of a lane's keys, for want of groups
+    constexpr int NE = HALF ? 1 : NG / WT;                      // groups whose exponentials a wave takes
+    constexpr int KE = HALF ? 4 : 8;                            // of them each lane's keys
     constexpr int DB = D / 128;                                 // 16-dimension blocks per wave
-    constexpr int VL = kKeyTile * (D / 8) / 128;                // 16-byte chunks of V per lane
+    constexpr int VL = kKeyTile * (D / 8) / (64 * WT);          // 16-byte chunks of V per lane
     constexpr int V_U16 = TC * kKeyTile * D, P_U16 = TC * NG * 2 * 512;
     constexpr int T = 512 / (16 * NG), BATCH = NG < 4 ? 4 * NG : 16;    // lanes per column's maxima
     static_assert(D % 128 == 0 && T >= 4 && T <= 32, "whole blocks per wave, whole lane groups per column");
     __shared__ __attribute__((aligned(16))) uint16_t lds[V_U16 + P_U16];
     __shared__ float smax[NG][16];
-    __shared__ float lred[NG][NG > 1 ? TC : 8][16];             // by tile, or tile and half
+    constexpr int LR = HALF ? 8 : TC;                           // column sums: by tile, or tile and half
+    __shared__ float lred[NG][LR][16];
     uint16_t *vt = lds, *pb = lds + V_U16;
     const int tid = threadIdx.x, l = tid & 63, j = l & 15, G = l >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wt = wave >> 1, wh = wave & 1;                    // exponentials and V: tile, half of it
+    const int wt = wave / WT, wh = wave % WT;                   // exponentials and V: tile, share of it
     const int wg = static_cast<int>(blockIdx.x), ng = a.sub, kvh0 = static_cast<int>(blockIdx.y) * ng;
     const uint64_t j0 = static_cast<uint64_t>(wg) * static_cast<uint64_t>(a.keys_pv);
     const uint64_t j1 = j0 + static_cast<uint64_t>(a.keys_pv) < a.n ? j0 + static_cast<uint64_t>(a.keys_pv) : a.n;
     const uint16_t *vbase = a.v + static_cast<uint64_t>(blockIdx.y) * a.kv_stride;
-    const int zb = NG > 1 ? NE * wh : 0, kb = NG > 1 ? 0 : KE * wh;  // this wave's first group, each lane's first key
+    const int zb = HALF ? 0 : NE * wh, kb = HALF ? KE * wh : 0;  // this wave's first group, each lane's first key
 
     f32x4 sc[NE][KE / 4];
     auto load_scores = [&](uint64_t c0) {
@@ -1420,7 +1426,7 @@ __global__ __launch_bounds__(512, 1) void decode_pv_groups(DecodeArgs a)
     for (int i = 0; i < NE; i++) {
         lsum[i] += __shfl_xor(lsum[i], 16);
         lsum[i] += __shfl_xor(lsum[i], 32);
-        if (G == 0) lred[zb + i][NG > 1 ? wt : wave][j] = lsum[i];
+        if (G == 0) lred[zb + i][HALF ? wave : wt][j] = lsum[i];
     }
     if (j < a.g) {
         const uint64_t zs = static_cast<uint64_t>(a.nwg_pv) * a.g;       // cells of a group
@@ -1437,7 +1443,7 @@ __global__ __launch_bounds__(512, 1) void decode_pv_groups(DecodeArgs a)
         if (z < ng && h < a.g) {
             float L = 0.0f;
 #pragma unroll
-            for (int t = 0; t < (NG > 1 ? TC : 8); t++) L += lred[z][t][h];
+            for (int t = 0; t < LR; t++) L += lred[z][t][h];
             if (a.sink_on && wg == 0) L += exp_poly(a.sink - smax[z][h]);    // once per column
             a.part_l[(static_cast<uint64_t>(kvh0 + z) * a.nwg_pv + wg) * a.g + h] = L;
         }

@@ -275,13 +275,17 @@ inline bool decode_pv_loop_ok(int d, int g, int rows, bool fused)
 // leaves the 256-key chunks of decode_pv one or two tiles over (`run` whole
 // tiles a workgroup), which costs those a whole chunk: one row at 32 769 and
 // 40 001 25.4 and 27.0 -> 24.5 and 26.4, but 49 153 and 131 072 (12 and 32
-// tiles) 29.7 and 55.9 -> 31.3 and 58.4. Runs past 2^25 tiles (2^30 keys) are
+// tiles) 29.7 and 55.9 -> 31.3 and 58.4. At D = 128 (chunks of 8 tiles) from
+// runs of 6 tiles on: 8 rows of 8 heads on 4 KV heads after 8 000 (4 tiles)
+// 23.7 us and 26.0 this way, after 16 000, 32 000 and 131 000 31.4, 51.5 and
+// 154 -> 28.6, 42.5 and 105. Runs past 2^25 tiles (2^30 keys) are
 // left to decode_pv.
-inline bool decode_pv_groups_dim(int d, int sub) { return d == 256 && sub >= 1 && sub <= kDecodeMaxSub; }
+inline bool decode_pv_groups_dim(int d, int sub) { return (d == 128 || d == 256) && sub >= 1 && sub <= kDecodeMaxSub; }
 inline bool decode_pv_groups_ok(int d, int sub, int g, uint64_t run)
 {
     const bool rest = run % 8 == 1 || run % 8 == 2;
-    return decode_pv_groups_dim(d, sub) && run <= (uint64_t{1} << 25) && (sub > 1 || g > 8 || (rest && run < 32));
+    return decode_pv_groups_dim(d, sub) && run <= (uint64_t{1} << 25) && (d == 256 || run >= 6) &&
+           (sub > 1 || g > 8 || (d == 256 && rest && run < 32));
 }
 // Its workgroups per KV head: one round of the compute units.
 inline uint64_t decode_pv_groups_wgs(uint64_t kv_heads, uint64_t cus) { return cus > kv_heads ? cus / kv_heads : 1; }

@@ -317,7 +317,7 @@ static hipError_t decode_dm(const DecodeArgs &a, int kv_heads, hipStream_t s)
     }
     if (a.pv_all) {
         // pass 2 over all the KV head's groups in one workgroup
-        if constexpr (D == 256) {
+        if constexpr (D == 128 || D == 256) {
             const dim3 gall(a.nwg_pv, kv_heads, 1);
             e = a.sub == 1   ? launch(decode_pv_groups<D, 1>, gall, dim3(512), s, a)
                 : a.sub == 2 ? launch(decode_pv_groups<D, 2>, gall, dim3(512), s, a)

@@ -1,6 +1,6 @@
 """GPU parity of pass 2 over all the groups of a KV head per workgroup
-(decode_pv_groups: head_dim 256, past one round of 256-key workgroups per
-group), at the edges of its runs and chunks: 1 to 8 groups (its instantiations
+(decode_pv_groups: head_dim 128 and 256, past one round of 256-key workgroups
+per group), at the edges of its runs and chunks: 1 to 8 groups (its instantiations
 hold 1, 2, 4 and 8), a group count below the instantiation's, padded columns,
 runs of 4 tiles and of one tile more than a chunk, a partial last tile and a
 last workgroup with less than the others, and the sink. 16 KV heads, so that a
@@ -17,7 +17,7 @@ from gpu_util import run_hsdpa
 pytestmark = pytest.mark.gpu
 
 CASES = [
-    # name, heads, kv_heads, rows, past, sink
+    # name, heads, kv_heads, rows, past, sink (head_dim 256)
     ("one_group_8_columns_9_tile_runs", 128, 16, 1, 4096, None),     # 129 tiles: one over 8 per run
     ("one_group_16_columns_partial_tile", 128, 16, 2, 4300, None),
     ("one_group_9_columns", 48, 16, 3, 8190, None),
@@ -35,13 +35,26 @@ CASES = [
 ]
 
 
-@pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
+# head_dim 128: runs of 6 tiles or more, chunks of 8 tiles up to 4 groups, of 4 beyond
+CASES_128 = [
+    ("d128_one_group_9_tile_runs", 128, 16, 2, 4300, None),
+    ("d128_two_groups_7_tile_runs", 128, 16, 4, 3100, None),
+    ("d128_three_groups_of_four", 128, 16, 6, 3300, None),
+    ("d128_four_groups_6_tile_runs", 128, 16, 8, 2900, None),
+    ("d128_four_groups_two_chunks", 32, 4, 8, 20011, None),
+    ("d128_eight_groups_6_tile_runs", 128, 16, 16, 2600, None),
+    ("d128_two_groups_sink", 128, 16, 4, 3100, 6.0),
+]
+ALL = [c + (256,) for c in CASES] + [c + (128,) for c in CASES_128]
+
+
+@pytest.mark.parametrize("case", ALL, ids=[c[0] for c in ALL])
 def test_groups_parity(torch_cuda, case):
-    name, h, kvh, rows, past, sink = case
+    name, h, kvh, rows, past, sink, dim = case
     import numpy as np
     import torch
 
-    w = W.make(name, heads=h, kv_heads=kvh, head_dim=256, rows=rows, past=past, seed=91)
+    w = W.make(name, heads=h, kv_heads=kvh, head_dim=dim, rows=rows, past=past, seed=91)
     plan = hsdpa.Plan(w.heads, w.gqa, w.head_dim, w.capacity, sink=sink is not None)
     print(f"case {name}", flush=True)
     if sink is None:
