@@ -29,6 +29,8 @@ struct hsdpa_plan {
     // split causal workspace (floats), after the decode's: partial row maxima,
     // outputs and sums of split_units (split, 32-row group, head) cells
     uint64_t split_units;
+    // the workspace without what plan_layout leaves out of a narrow one
+    bool narrow;
     uint64_t off_smax, off_so, off_sl;
     uint64_t ws_bytes;
 };
@@ -389,10 +391,12 @@ DecodeCfg decode_cfg(const hsdpa_plan *p, uint64_t rows, uint64_t n, int sub, bo
     // the groups of a KV head in each workgroup, in one round of runs of whole
     // tiles (decode_pv_groups_ok)
     if (!fused && groups * nch > cu1) {
-        const uint64_t per = hsdpa::decode_pv_groups_wgs(p->kv_heads, cu1);
+        // (a narrow workspace may hold fewer)
+        const uint64_t wgs = hsdpa::decode_pv_groups_wgs(p->kv_heads, cu1);
+        const uint64_t per = std::min(wgs, p->dec_part / (static_cast<uint64_t>(sub) * static_cast<uint64_t>(c.g)));
         const uint64_t tiles = (n + hsdpa::kKeyTile - 1) / hsdpa::kKeyTile;
-        const uint64_t run = std::max<uint64_t>((tiles + per - 1) / per, 4);
-        if (hsdpa::decode_pv_groups_ok(d, sub, c.g, run)) {
+        const uint64_t run = per ? std::max<uint64_t>((tiles + per - 1) / per, 4) : 0;
+        if (2 * per >= wgs && hsdpa::decode_pv_groups_ok(d, sub, c.g, run)) {
             c.keys_pv = static_cast<int>(run) * hsdpa::kKeyTile;
             c.pv_all = 1;
         }
@@ -428,9 +432,9 @@ uint64_t decode_nwg_pv_max(const hsdpa_plan *p, uint64_t rows, int sub)
     // 128 keys each
     uint64_t all = 0;
     const uint64_t per_all = hsdpa::decode_pv_groups_wgs(p->kv_heads, static_cast<uint64_t>(p->cus));
-    if (hsdpa::decode_pv_groups_dim(d, sub)) {
+    if (!p->narrow && hsdpa::decode_pv_groups_dim(d, sub)) {
         all = std::min(by128, per_all);
-        if (p->form != HSDPA_FORM_FUSED && (sub > 1 || g > 8)) return all;
+        if (p->form != HSDPA_FORM_FUSED && (sub > 1 || g > 8)) return std::max(all, one_round);
     }
     // the chunked pass 2 gives way to 256-key workgroups where it cannot run
     // (decode_pv_loop_ok) or a run would exceed 2^30 keys
@@ -440,6 +444,9 @@ uint64_t decode_nwg_pv_max(const hsdpa_plan *p, uint64_t rows, int sub)
                       (p->form != HSDPA_FORM_FUSED || hsdpa::decode_pv_loop_ok(d, g, static_cast<int>(rows), true));
     if (!loop || run_max > (uint64_t{1} << 30))
         return std::max({all, one_round, by256});
+    // several rows at D = 256 in a narrow workspace: 256-key workgroups' worth
+    // (for any past with more than 4 groups; up to CUs / kv_heads of them)
+    if (d == 256 && rows > 1 && sub > 1) return std::max({all, one_round, sub > 4 ? by256 : std::min(by256, per_all)});
     return std::max(all, one_round);
 }
 
@@ -466,48 +473,13 @@ struct Part {
 
 }  // namespace
 
-hsdpa_status hsdpa_plan_create(const hsdpa_spec *spec, hsdpa_plan **out)
+// The plan's workspace for `cols` decode columns per KV head. narrow: without
+// the partials that pass 2 over all groups and the equal shares of the causal
+// prefill take beyond the other forms' (their calls then take those).
+static void plan_layout(hsdpa_plan *p, uint64_t cols, bool narrow)
 {
-    if (!spec || !out) return HSDPA_ERR_NULL;
-    *out = nullptr;
-    const hsdpa_status st = check_spec(*spec);
-    if (st != HSDPA_OK) return st;
-    hsdpa_plan *p = new (std::nothrow) hsdpa_plan();
-    if (!p) return HSDPA_ERR_HIP;
-    p->spec = *spec;
-    const uint64_t d = spec->head_dim, g = spec->gqa, kvh = spec->heads / spec->gqa;
-    const uint64_t cap = spec->kv_capacity;
-    p->kv_heads = kvh;
-    // the Fused form declines the sink (src/jit/emit_sdpa.rs:468-470) and the
-    // engine then emits the Chained one
-    p->form = spec->form == HSDPA_FORM_FUSED && d <= 256 && !spec->sink ? HSDPA_FORM_FUSED : HSDPA_FORM_CHAINED;
-    if (p->form == HSDPA_FORM_FUSED && g > kFusedMaxGqa) {
-        delete p;
-        return HSDPA_ERR_FORM;
-    }
-    p->max_rows = spec->max_rows ? spec->max_rows : cap;
-    // the grids (and so the workspace) follow the device's compute units; with
-    // no device current, the MI355X's 256
-    int cus = 0;
-    const bool on_gfx950 = check_device(&cus) == HSDPA_OK;
-    p->cus = on_gfx950 && cus > 0 ? cus : 256;
-    // the static scratch's address on this device, so that no call of
-    // hsdpa_attention_static (possibly under graph capture) looks it up
-    if (on_gfx950) {
-        void *scratch = nullptr;
-        if (hsdpa::static_scratch(&scratch) != hipSuccess) {
-            delete p;
-            return HSDPA_ERR_HIP;
-        }
-    }
-    // decode columns: the query heads of one row, or up to 16 rows of them
-    const int gi = static_cast<int>(std::min<uint64_t>(g, 1u << 20));
-    const bool pad_ok = hsdpa::decode_rows_ok(static_cast<int>(d)) && hsdpa::decode_groups_pad(gi) > 0;
-    uint64_t cols = hsdpa::decode_groups(gi) || pad_ok ? g : 0;
-    if (hsdpa::decode_rows_ok(static_cast<int>(d)) && p->max_rows > 1) {
-        const uint64_t mr = std::min<uint64_t>(hsdpa::kDecodeMaxRows, p->max_rows);
-        cols = std::max(cols, std::min<uint64_t>(hsdpa::kDecodeMaxCols, mr * g));
-    }
+    const uint64_t d = p->spec.head_dim, g = p->spec.gqa, kvh = p->kv_heads, cap = p->spec.kv_capacity;
+    p->narrow = narrow;
     p->dec_cols = cols;
     p->dec_npad = align_up(cap, hsdpa::kDecodeKeysPV);
     p->dec_nwg_qk = (cap + hsdpa::kDecodeKeysQK - 1) / hsdpa::kDecodeKeysQK;
@@ -558,6 +530,57 @@ hsdpa_status hsdpa_plan_create(const hsdpa_spec *spec, hsdpa_plan **out)
     p->off_sl = off;
     off = align_up(off + cells * 4, kAlign);
     p->ws_bytes = off;
+}
+
+hsdpa_status hsdpa_plan_create(const hsdpa_spec *spec, hsdpa_plan **out)
+{
+    if (!spec || !out) return HSDPA_ERR_NULL;
+    *out = nullptr;
+    const hsdpa_status st = check_spec(*spec);
+    if (st != HSDPA_OK) return st;
+    hsdpa_plan *p = new (std::nothrow) hsdpa_plan();
+    if (!p) return HSDPA_ERR_HIP;
+    p->spec = *spec;
+    const uint64_t d = spec->head_dim, g = spec->gqa, kvh = spec->heads / spec->gqa;
+    const uint64_t cap = spec->kv_capacity;
+    p->kv_heads = kvh;
+    // the Fused form declines the sink (src/jit/emit_sdpa.rs:468-470) and the
+    // engine then emits the Chained one
+    p->form = spec->form == HSDPA_FORM_FUSED && d <= 256 && !spec->sink ? HSDPA_FORM_FUSED : HSDPA_FORM_CHAINED;
+    if (p->form == HSDPA_FORM_FUSED && g > kFusedMaxGqa) {
+        delete p;
+        return HSDPA_ERR_FORM;
+    }
+    p->max_rows = spec->max_rows ? spec->max_rows : cap;
+    // the grids (and so the workspace) follow the device's compute units; with
+    // no device current, the MI355X's 256
+    int cus = 0;
+    const bool on_gfx950 = check_device(&cus) == HSDPA_OK;
+    p->cus = on_gfx950 && cus > 0 ? cus : 256;
+    // the static scratch's address on this device, so that no call of
+    // hsdpa_attention_static (possibly under graph capture) looks it up
+    if (on_gfx950) {
+        void *scratch = nullptr;
+        if (hsdpa::static_scratch(&scratch) != hipSuccess) {
+            delete p;
+            return HSDPA_ERR_HIP;
+        }
+    }
+    // decode columns: the query heads of one row, or up to 16 rows of them
+    const int gi = static_cast<int>(std::min<uint64_t>(g, 1u << 20));
+    const bool pad_ok = hsdpa::decode_rows_ok(static_cast<int>(d)) && hsdpa::decode_groups_pad(gi) > 0;
+    uint64_t cols = hsdpa::decode_groups(gi) || pad_ok ? g : 0;
+    if (hsdpa::decode_rows_ok(static_cast<int>(d)) && p->max_rows > 1) {
+        const uint64_t mr = std::min<uint64_t>(hsdpa::kDecodeMaxRows, p->max_rows);
+        cols = std::max(cols, std::min<uint64_t>(hsdpa::kDecodeMaxCols, mr * g));
+    }
+    // within the static scratch where the narrow workspace is (a plan that
+    // hsdpa_attention_static takes), otherwise as the kernels run fastest
+    plan_layout(p, cols, false);
+    if (p->ws_bytes > HSDPA_STATIC_SCRATCH_BYTES) {
+        plan_layout(p, cols, true);
+        if (p->ws_bytes > HSDPA_STATIC_SCRATCH_BYTES) plan_layout(p, cols, false);
+    }
     *out = p;
     return HSDPA_OK;
 }
