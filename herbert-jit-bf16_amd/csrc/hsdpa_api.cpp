@@ -28,7 +28,7 @@ struct hsdpa_plan {
     uint64_t off_scores, off_wgmax, off_part_o, off_part_l, off_bmax, off_part_x, off_fcfg, dec_bytes;
     // split causal workspace (floats), after the decode's: partial row maxima,
     // outputs and sums of split_units (split, 32-row group, head) cells
-    uint64_t split_units;
+    uint64_t split_units, flat_units;
     // the workspace without what plan_layout leaves out of a narrow one
     bool narrow;
     uint64_t off_smax, off_so, off_sl;
@@ -522,9 +522,13 @@ static void plan_layout(hsdpa_plan *p, uint64_t cols, bool narrow)
     for (uint64_t r = 1; r <= std::min<uint64_t>(hsdpa::kDecodeMaxRows + 8, p->max_rows) && !causal; r++)
         causal = reaches_causal(p, r);
     p->split_units = causal ? std::min<uint64_t>(hsdpa::kSplitUnits, 8 * static_cast<uint64_t>(p->cus)) : 0;
-    const uint64_t cells = p->split_units * 32;
+    // (the equal shares at D = 128: two cells a workgroup)
+    p->flat_units = narrow || cap <= hsdpa::kFlatMinLongest * hsdpa::kKeyTile
+                        ? p->split_units
+                        : hsdpa::prefill_flat_units(static_cast<int>(d), p->split_units);
+    const uint64_t cells = p->flat_units * 32;
     p->off_smax = off;
-    off = align_up(off + p->split_units * hsdpa::kSplitMaxCells * 4, kAlign);
+    off = align_up(off + p->flat_units * hsdpa::kSplitMaxCells * 4, kAlign);
     p->off_so = off;
     off = align_up(off + cells * d * 4, kAlign);
     p->off_sl = off;
@@ -684,6 +688,7 @@ static hsdpa_status run_part(const hsdpa_plan *plan, const hsdpa_call *call, con
         ps.sl = reinterpret_cast<float *>(ws + plan->off_sl);
     }
     ps.units = plan->split_units;
+    ps.flat_units = plan->flat_units;
     ps.cus = plan->cus;
     // a chunk the one-workgroup causal kernel would spread too thin (it would be
     // split over its keys) and whose row blocks see few key tiles: the waves
@@ -704,10 +709,16 @@ static hsdpa_status run_part(const hsdpa_plan *plan, const hsdpa_call *call, con
     }
     const int sp = hsdpa::prefill_split_count(a, d, static_cast<int>(s.heads), ps);
     const bool paired = sp == 1 && hsdpa::prefill_pair_rows(a, d, static_cast<int>(s.heads), ps).srows > 0;
+    // the equal shares are a split over the keys, or (where pairs of row groups
+    // would do) those row groups evened out further
+    hsdpa::FlatShape flat_shape;
+    const bool flat = hsdpa::prefill_flat_shape(a, d, static_cast<int>(s.heads), ps, flat_shape);
     if (kernels)
-        *kernels = sp > 1 ? HSDPA_KERNELS_CAUSAL_SPLIT : paired ? HSDPA_KERNELS_CAUSAL_PAIRED : HSDPA_KERNELS_CAUSAL;
-    if (splits) *splits = static_cast<uint32_t>(sp);
-    if (launches) *launches += sp > 1 || paired ? 3 : 1;
+        *kernels = paired ? HSDPA_KERNELS_CAUSAL_PAIRED
+                   : sp > 1 || flat ? HSDPA_KERNELS_CAUSAL_SPLIT
+                                    : HSDPA_KERNELS_CAUSAL;
+    if (splits) *splits = static_cast<uint32_t>(flat && !paired && sp == 1 ? 2 : sp);
+    if (launches) *launches += sp > 1 || paired || flat ? 3 : 1;
     if (!launch) return HSDPA_OK;
     const hipError_t e = hsdpa::launch_prefill(a, d, static_cast<int>(s.heads), ps, st);
     return e == hipSuccess ? HSDPA_OK : HSDPA_ERR_HIP;

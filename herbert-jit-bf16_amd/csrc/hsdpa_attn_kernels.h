@@ -1870,6 +1870,50 @@ __device__ __forceinline__ void store_rows(const f32x16 *o, uint16_t *op, const 
         }
 }
 
+// The row maxima (of the unscaled dot products) over the tiles [tb, te) of one
+// row block's key range, in the lanes of each half wave; the walk is pv_walk's.
+template <int D, int NW>
+__device__ __forceinline__ float max_walk(const PrefillArgs &a, const uint16_t *kg, uint16_t (*kb)[kKeyTile * Pad<D>::K],
+                                          const u32x4 (&qb)[D / 16], uint64_t lim, int nfull, int tb, int te, int tid)
+{
+    constexpr int THREADS = 64 * NW, SK = Pad<D>::K;
+    const int l = tid & 63, col = l & 31, grp = l >> 5;
+    const int arow = swap23(col) * SK + 8 * grp;
+    u32x4 kr[Tile<D, THREADS>::kPer];
+    tile_gload<D, THREADS, false>(kg, static_cast<uint64_t>(tb) * kKeyTile, a.n, tid, kr);
+    tile_lstore_padded<D, THREADS>(kb[0], SK, tid, kr);
+    __syncthreads();
+    float m = kNegInf;
+    // the next tile's load is not branched around (past the cache it reads row
+    // 0, unused)
+    for (int t = tb; t < te; t++) {
+        const uint64_t t0 = static_cast<uint64_t>(t) * kKeyTile;
+        tile_gload<D, THREADS, false>(kg, t0 + kKeyTile, a.n, tid, kr);
+        __builtin_amdgcn_sched_barrier(0);
+        const uint16_t *kt = kb[(t - tb) & 1];
+        f32x16 acc = {};
+#pragma unroll
+        for (int s = 0; s < D / 16; s += 2) {
+            // two K operands requested before their MFMAs
+            const u32x4 k0 = load16(kt + arow + 16 * s), k1 = load16(kt + arow + 16 * (s + 1));
+            acc = mfma(k0, qb[s], acc);
+            acc = mfma(k1, qb[s + 1], acc);
+        }
+        if (t < nfull) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) m = __builtin_fmaxf(m, acc[r]);
+        } else {
+            const int vis = static_cast<int>(static_cast<int64_t>(lim) - static_cast<int64_t>(t0));
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+                if (key_of(r, grp) <= vis) m = __builtin_fmaxf(m, acc[r]);
+        }
+        if (t + 1 < te) tile_lstore_padded<D, THREADS>(kb[(t - tb + 1) & 1], SK, tid, kr);
+        __syncthreads();
+    }
+    return m;
+}
+
 // The tiles [tb, te) of one row block's key range: scores, exponentials at the
 // exact maximum and P.V with P = hi + lo, added to o and lsum. K rows past the
 // cache read row 0 and are never visible, V rows past it are zeroed. Every
@@ -2667,7 +2711,7 @@ struct SplitSegs {
 template <int D, int HPW, int NW, bool PAIRED = false>
 __global__ __launch_bounds__(64 * NW, 1) void prefill_split_max(PrefillArgs a, SplitArgs sp)
 {
-    constexpr int RB = NW / HPW, THREADS = 64 * NW;
+    constexpr int RB = NW / HPW;
     constexpr int SK = Pad<D>::K;
     __shared__ __attribute__((aligned(16))) uint16_t kb[2][kKeyTile * SK];
     const int tid = threadIdx.x;
@@ -2677,7 +2721,6 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_split_max(PrefillArgs a, S
     const int kvh = head / a.gqa;
     const SplitSegs<PAIRED> segs(a, sid, 32 * RB);
     const uint16_t *kg = a.k + static_cast<uint64_t>(kvh) * a.kv_stride;
-    const int arow = swap23(col) * SK + 8 * grp;
     // one key range, then (paired) the second: the body is instantiated for
     // each, so that no register stays live from one to the other
     auto run = [&](const SplitSeg sg) {
@@ -2690,7 +2733,6 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_split_max(PrefillArgs a, S
         const uint64_t lim = a.past + row;
         const int tb = sg.tb, te = sg.te;
 
-        u32x4 kr[Tile<D, THREADS>::kPer];
         u32x4 qb[D / 16];
         const uint16_t *qp = a.q + (rowv ? row : 0) * a.q_row + static_cast<uint64_t>(head) * a.q_head;
 #pragma unroll
@@ -2699,38 +2741,7 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_split_max(PrefillArgs a, S
             qb[s] = q_chunk(v, rowv, q_sign(a));
         }
         float m = kNegInf;
-        if (tb < te) {
-            tile_gload<D, THREADS, false>(kg, static_cast<uint64_t>(tb) * kKeyTile, a.n, tid, kr);
-            tile_lstore_padded<D, THREADS>(kb[0], SK, tid, kr);
-            __syncthreads();
-            // as prefill_attn's pass 1: the next tile's load is not branched
-            // around (past the cache it reads row 0, unused)
-            for (int t = tb; t < te; t++) {
-                const uint64_t t0 = static_cast<uint64_t>(t) * kKeyTile;
-                tile_gload<D, THREADS, false>(kg, t0 + kKeyTile, a.n, tid, kr);
-                __builtin_amdgcn_sched_barrier(0);
-                const uint16_t *kt = kb[(t - tb) & 1];
-                f32x16 acc = {};
-#pragma unroll
-                for (int s = 0; s < D / 16; s += 2) {
-                    // two K operands requested before their MFMAs
-                    const u32x4 k0 = load16(kt + arow + 16 * s), k1 = load16(kt + arow + 16 * (s + 1));
-                    acc = mfma(k0, qb[s], acc);
-                    acc = mfma(k1, qb[s + 1], acc);
-                }
-                if (t < nfull) {
-#pragma unroll
-                    for (int r = 0; r < 16; r++) m = __builtin_fmaxf(m, acc[r]);
-                } else {
-                    const int vis = static_cast<int>(static_cast<int64_t>(lim) - static_cast<int64_t>(t0));
-#pragma unroll
-                    for (int r = 0; r < 16; r++) 
-                        if (key_of(r, grp) <= vis) m = __builtin_fmaxf(m, acc[r]);
-                }
-                if (t + 1 < te) tile_lstore_padded<D, THREADS>(kb[(t - tb + 1) & 1], SK, tid, kr);
-                __syncthreads();
-            }
-        }
+        if (tb < te) m = max_walk<D, NW>(a, kg, kb, qb, lim, nfull, tb, te, tid);
         m = __builtin_fmaxf(m, __shfl_xor(m, 32));
         const int slot = sg.slot < 0 ? 0 : sg.slot;
         if (rowv && grp == 0) sp.smax[(static_cast<uint64_t>(slot) * sp.heads + head) * a.rows + row] = m;

@@ -116,6 +116,7 @@ struct PrefillSplit {
     float *smax, *so, *sl;
     uint64_t units;
     int cus;
+    uint64_t flat_units;    // the same for the equal shares (prefill_flat), at least units
 };
 constexpr uint64_t kSplitMaxCells = 128;
 
@@ -376,12 +377,13 @@ __host__ __device__ inline uint64_t pair_share(uint64_t ti, uint64_t tj)
 constexpr uint64_t kPairMinLongest = 64;
 struct PairRows {
     uint64_t r0, srows;
+    uint64_t longest;       // the tiles of its longest workgroup
 };
 
 inline PairRows prefill_pairs(const PrefillArgs &a, uint64_t R, uint64_t wgs, uint64_t rpw, int heads,
                               const PrefillSplit &ps)
 {
-    const PairRows none{0, 0};
+    const PairRows none{0, 0, 0};
     if (ps.units == 0 || ps.cus <= 0 || R < 2 || wgs > static_cast<uint64_t>(ps.cus)) return none;
     uint64_t longest = R % 2 ? causal_tiles(a.past, a.rows, R / 2, rpw) : 0, split = 0;
     for (uint64_t i = 0; i < R - 1 - i; i++) {
@@ -396,7 +398,57 @@ inline PairRows prefill_pairs(const PrefillArgs &a, uint64_t R, uint64_t wgs, ui
     const uint64_t r0 = (R - split) * rpw, srows = a.rows - r0;
     const uint64_t h = static_cast<uint64_t>(heads);
     if (2 * srows * h > ps.units * 32 || 2 * a.rows * h > ps.units * kSplitMaxCells) return none;
-    return PairRows{r0, srows};
+    return PairRows{r0, srows, longest};
 }
+
+// The causal prefill in equal shares (hsdpa_prefill_flat.hip): the tiles of R
+// row groups (8 / HPW blocks of 32 rows, HPW = 2^lh query heads) for each of
+// the head groups, one after the other, T in all, Th a head group, cut into wm
+// (row maxima) and wp (P.V) parts.
+struct FlatShape {
+    float *smax, *so, *sl;
+    uint32_t T, Th, R, p0, last, lh, heads, wm, wp; // row group rg has p0 + (rg + 1) 8 / HPW tiles, the last `last`
+};
+// Workspace for them: cells of 8 waves x 32 rows, two a workgroup.
+constexpr int kFlatDim = 128;
+inline uint64_t prefill_flat_units(int d, uint64_t units) { return d == kFlatDim ? 2 * units : units; }
+// Whether the equal shares take a call whose grid's longest workgroup walks
+// `longest` tiles (0: more than one round of them; row group by row group, in
+// pairs or split): where a share, with three tiles for its second row group's
+// start, is an eighth shorter, the longest row group sees more than
+// kFlatMinLongest tiles (as for kPairMinLongest, fewer than which do not pay
+// two more launches), and the workspace holds the parts. 1800 rows of 32/8
+// heads with no cache 131.4 -> 117.6 us, 700 after 900 with the sink 78.4 ->
+// 68.4; calls that fill their round already stay as they were.
+constexpr uint64_t kFlatMinLongest = 40;
+inline bool prefill_flat(const PrefillArgs &a, int d, int heads, const PrefillSplit &ps, uint64_t longest, FlatShape &f)
+{
+    if (d != kFlatDim || longest == 0 || ps.cus <= 0) return false;
+    const uint64_t cus = static_cast<uint64_t>(ps.cus), h = static_cast<uint64_t>(heads);
+    f.lh = a.gqa % 8 == 0 ? 3 : a.gqa % 4 == 0 ? 2 : a.gqa % 2 == 0 ? 1 : 0;
+    const uint64_t RB = 8u >> f.lh, R = (a.rows + 32 * RB - 1) / (32 * RB);
+    const uint64_t p0 = (a.past + kKeyTile - 1) / kKeyTile, last = (a.past + a.rows + kKeyTile - 1) / kKeyTile;
+    if (last <= kFlatMinLongest || last > (1u << 20) || R > (1u << 12)) return false;
+    const uint64_t Th = (R - 1) * p0 + RB * ((R - 1) * R / 2) + last, T = Th * (h >> f.lh);
+    const uint64_t wp = cus, wm = 2 * cus;                      // the maxima's registers allow two per unit
+    if ((T + 1) * wm > 0xFFFFFFFFull || T < 4 * wm || 8 * (T / cus + 3) > 7 * longest) return false;
+    if (a.rows * h > 0x7FFFFFFFull || 16 * wp > ps.flat_units) return false;
+    if ((last / (T / wm) + 2) * h * a.rows > ps.flat_units * kSplitMaxCells) return false;
+    f.smax = ps.smax;
+    f.so = ps.so;
+    f.sl = ps.sl;
+    f.T = static_cast<uint32_t>(T);
+    f.Th = static_cast<uint32_t>(Th);
+    f.R = static_cast<uint32_t>(R);
+    f.p0 = static_cast<uint32_t>(p0);
+    f.last = static_cast<uint32_t>(last);
+    f.heads = static_cast<uint32_t>(heads);
+    f.wm = static_cast<uint32_t>(wm);
+    f.wp = static_cast<uint32_t>(wp);
+    return true;
+}
+hipError_t launch_prefill_flat(const PrefillArgs &a, const FlatShape &f, hipStream_t s);
+// the equal shares' shape for a call launch_prefill would run so
+bool prefill_flat_shape(const PrefillArgs &a, int head_dim, int heads, const PrefillSplit &ps, FlatShape &f);
 
 }  // namespace hsdpa

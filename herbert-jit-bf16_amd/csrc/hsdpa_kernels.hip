@@ -396,8 +396,20 @@ int prefill_split_count(const PrefillArgs &a, int head_dim, int heads, const Pre
 PairRows prefill_pair_rows(const PrefillArgs &a, int head_dim, int heads, const PrefillSplit &ps)
 {
     const dim3 g = prefill_grid(a, head_dim, heads);
-    if (prefill_splits(a, static_cast<uint64_t>(g.x) * g.y, heads, ps) > 1) return PairRows{0, 0};
+    if (prefill_splits(a, static_cast<uint64_t>(g.x) * g.y, heads, ps) > 1) return PairRows{0, 0, 0};
     return prefill_pairs(a, g.x, static_cast<uint64_t>(g.x) * g.y, prefill_rows_per_wg(a, head_dim), heads, ps);
+}
+
+bool prefill_flat_shape(const PrefillArgs &a, int head_dim, int heads, const PrefillSplit &ps, FlatShape &f)
+{
+    if (head_dim != kFlatDim || ps.flat_units == 0) return false;
+    const dim3 g = prefill_grid(a, head_dim, heads);
+    const uint64_t tiles = (a.past + a.rows + kKeyTile - 1) / kKeyTile;
+    const uint64_t splits = static_cast<uint64_t>(prefill_split_count(a, head_dim, heads, ps));
+    const PairRows pr = prefill_pair_rows(a, head_dim, heads, ps);
+    const bool one_round = static_cast<uint64_t>(g.x) * g.y <= static_cast<uint64_t>(ps.cus);
+    const uint64_t longest = splits > 1 ? (tiles + splits - 1) / splits : pr.srows ? pr.longest : one_round ? tiles : 0;
+    return prefill_flat(a, head_dim, heads, ps, longest, f);
 }
 
 template <int D, int HPW>
@@ -447,6 +459,8 @@ hipError_t launch_gate(const GateArgs &a, hipStream_t s)
 
 hipError_t launch_prefill(const PrefillArgs &a, int head_dim, int heads, const PrefillSplit &ps, hipStream_t s)
 {
+    FlatShape f;
+    if (prefill_flat_shape(a, head_dim, heads, ps, f)) return launch_prefill_flat(a, f, s);
     if (a.sink_on) return launch_prefill_sink(a, head_dim, heads, ps, s);
     switch (head_dim) {
     case 64: return prefill_d<64>(a, heads, ps, s);

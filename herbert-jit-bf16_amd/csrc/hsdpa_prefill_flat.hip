@@ -1,5 +1,5 @@
-// hsdpa_prefill_flat.hip — the causal prefill in equal shares, head dimensions
-// up to 128: the key tiles of all (head group, row group) pairs of a call form
+// hsdpa_prefill_flat.hip — the causal prefill in equal shares at head
+// dimension 128: the key tiles of all (head group, row group) pairs of a call form
 // one sequence, and each workgroup of one round walks an equal part of it,
 // whatever the row groups' lengths. Where a grid of row groups, or an even
 // split of each, leaves compute units idle or waiting for the longest row
@@ -7,10 +7,11 @@
 // Three launches like the split form's: the row maxima, P.V at the exact
 // maximum, and a combine of the row groups that several workgroups share. Same
 // tile walks and numerics as prefill_attn; heads per workgroup and the sink are
-// arguments here, so that each head dimension has one instantiation. Larger
-// head dimensions keep the grids that start every workgroup at tile 0: their
-// KV heads do not fit an XCD's L2, which then serves the workgroups that walk
-// the same tiles at the same time.
+// arguments here, so that there is one instantiation. At D = 256 the grids that
+// start every workgroup at tile 0 stay: a KV head does not fit an XCD's L2,
+// which then serves the workgroups that walk the same tiles at the same time.
+// At the smaller head dimensions the shares' parts would take plans past the
+// static scratch that fit it.
 
 #include "hsdpa_attn_kernels.h"
 
@@ -182,25 +183,15 @@ __global__ __launch_bounds__(CombineShape<D>::THREADS) void flat_combine(Prefill
     combine_store<D>(a, row, head, t, o, L);
 }
 
-template <int D> static hipError_t flat_d(const PrefillArgs &a, const FlatShape &f, hipStream_t s)
+hipError_t launch_prefill_flat(const PrefillArgs &a, const FlatShape &f, hipStream_t s)
 {
+    constexpr int D = kFlatDim, CELLS = CombineShape<D>::CELLS;
     hipError_t e = launch(flat_max<D>, dim3(f.wm), dim3(64 * kFlatNW), s, a, f);
     if (e == hipSuccess) e = launch(flat_pv<D>, dim3(f.wp), dim3(64 * kFlatNW), s, a, f);
     if (e != hipSuccess) return e;
     const uint64_t cells = a.rows * f.heads;
-    return launch(flat_combine<D>, dim3(static_cast<unsigned>((cells + CombineShape<D>::CELLS - 1) / CombineShape<D>::CELLS)),
+    return launch(flat_combine<D>, dim3(static_cast<unsigned>((cells + CELLS - 1) / CELLS)),
                   dim3(CombineShape<D>::THREADS), s, a, f);
-}
-
-hipError_t launch_prefill_flat(const PrefillArgs &a, int head_dim, const FlatShape &f, hipStream_t s)
-{
-    switch (head_dim) {
-    case 32: return flat_d<32>(a, f, s);
-    case 64: return flat_d<64>(a, f, s);
-    case 96: return flat_d<96>(a, f, s);
-    case 128: return flat_d<128>(a, f, s);
-    default: return hipErrorInvalidValue;
-    }
 }
 
 }  // namespace hsdpa
