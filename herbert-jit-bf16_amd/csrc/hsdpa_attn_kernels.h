@@ -1919,8 +1919,10 @@ __device__ __forceinline__ float max_walk(const PrefillArgs &a, const uint16_t *
 // cache read row 0 and are never visible, V rows past it are zeroed. Every
 // wave of the workgroup walks the same tiles; a wave's tiles from nfull on
 // take the masked path.
-template <int D, int NW>
+// FETCHED: the caller has requested tile tb's K and V (into kr and vr).
+template <int D, int NW, bool FETCHED>
 __device__ __forceinline__ void pv_walk(const PrefillArgs &a, const uint16_t *kg, const uint16_t *vg,
+                                        u32x4 (&kr)[Tile<D, 64 * NW>::kPer], u32x4 (&vr)[Tile<D, 64 * NW>::kPer],
                                         uint16_t (*kb)[kKeyTile * Pad<D>::K], uint16_t (*vb)[kKeyTile * Pad<D>::V],
                                         const u32x4 (&qb)[D / 16], const RowExp &ex, uint64_t lim, int nfull, int tb,
                                         int te, int tid, f32x16 (&o)[D / 32], float &lsum)
@@ -1929,9 +1931,10 @@ __device__ __forceinline__ void pv_walk(const PrefillArgs &a, const uint16_t *kg
     constexpr int SK = Pad<D>::K, SV = Pad<D>::V;
     const int l = tid & 63, col = l & 31, grp = l >> 5;
     const int arow = swap23(col) * SK + 8 * grp;
-    u32x4 kr[Tile<D, THREADS>::kPer], vr[Tile<D, THREADS>::kPer];
-    tile_gload<D, THREADS, false>(kg, static_cast<uint64_t>(tb) * kKeyTile, a.n, tid, kr);
-    tile_gload<D, THREADS, false>(vg, static_cast<uint64_t>(tb) * kKeyTile, a.n, tid, vr);
+    if constexpr (!FETCHED) {
+        tile_gload<D, THREADS, false>(kg, static_cast<uint64_t>(tb) * kKeyTile, a.n, tid, kr);
+        tile_gload<D, THREADS, false>(vg, static_cast<uint64_t>(tb) * kKeyTile, a.n, tid, vr);
+    }
     // The next K tile is loaded first, the next V tile after the first half's
     // exponentials, so that their staging registers are not live at the peak;
     // the loads are not branched around, the masked and unmasked halves of a
@@ -2019,7 +2022,7 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_attn(PrefillArgs a)
 
     const uint16_t *kg = a.k + static_cast<uint64_t>(kvh) * a.kv_stride;
     const uint16_t *vg = a.v + static_cast<uint64_t>(kvh) * a.kv_stride;
-    u32x4 kr[Tile<D, THREADS>::kPer];
+    u32x4 kr[Tile<D, THREADS>::kPer], vr[Tile<D, THREADS>::kPer];
     u32x4 qb[D / 16];
     const uint16_t *qp = a.q + (rowv ? row : 0) * a.q_row + static_cast<uint64_t>(head) * a.q_head;
 #pragma unroll
@@ -2056,7 +2059,8 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_attn(PrefillArgs a)
     for (int t = 0; t < ntiles; t++) {
         const uint64_t t0 = static_cast<uint64_t>(t) * kKeyTile;
         const bool last = t + 1 == ntiles;
-        tile_gload<D, THREADS, false>(kg, t0 + kKeyTile, a.n, tid, kr);   // past the cache: row 0, unused
+        tile_gload<D, THREADS, false>(kg, last ? 0 : t0 + kKeyTile, a.n, tid, kr);   // after the last: pass 2's first tile
+        if (last) tile_gload<D, THREADS, false>(vg, 0, a.n, tid, vr);
         __builtin_amdgcn_sched_barrier(0);
         const f32x16 acc = qk(kb[t & 1]);
         if (t < nfull) {
@@ -2083,7 +2087,7 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_attn(PrefillArgs a)
     // the sink's exponential starts the row's sum (in one of its two lanes),
     // so that nothing of it stays live across the tiles
     float lsum = SINK && grp == 0 ? exp_poly(a.sink - ms) : 0.0f;
-    pv_walk<D, NW>(a, kg, vg, kb, vb, qb, ex, lim, nfull, 0, ntiles, tid, o, lsum);
+    pv_walk<D, NW, true>(a, kg, vg, kr, vr, kb, vb, qb, ex, lim, nfull, 0, ntiles, tid, o, lsum);
     lsum += __shfl_xor(lsum, 32);
     if (rowv) {
         uint16_t *op = a.out + row * a.out_row + static_cast<uint64_t>(head) * D;
@@ -2800,7 +2804,8 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_split_pv(PrefillArgs a, Sp
         // the sink's exponential, once per row: it starts the sum of the whole
         // range's or of slot 0's (in one lane of two)
         float lsum = SINK && (DIRECT || sg.slot == 0) && grp == 0 ? exp_poly(a.sink - ms) : 0.0f;
-        if (tb < te) pv_walk<D, NW>(a, kg, vg, kb, vb, qb, ex, lim, nfull, tb, te, tid, o, lsum);
+        u32x4 kr[Tile<D, 64 * NW>::kPer], vr[Tile<D, 64 * NW>::kPer];
+        if (tb < te) pv_walk<D, NW, false>(a, kg, vg, kr, vr, kb, vb, qb, ex, lim, nfull, tb, te, tid, o, lsum);
         lsum += __shfl_xor(lsum, 32);
         if (!rowv) return;
         if constexpr (DIRECT) {

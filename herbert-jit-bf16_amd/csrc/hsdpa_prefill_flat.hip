@@ -136,7 +136,8 @@ __global__ __launch_bounds__(64 * kFlatNW, 1) void flat_pv(PrefillArgs a, FlatSh
         for (int dt = 0; dt < D / 32; dt++) o[dt] = f32x16{};
         // the sink's exponential, once per row: in its first part
         float lsum = a.sink_on && k.tb == 0 && grp == 0 ? exp_poly(a.sink - ms) : 0.0f;
-        pv_walk<D, kFlatNW>(a, a.k + kv, a.v + kv, kb, vb, r.qb, ex, r.lim, r.nfull, static_cast<int>(k.tb),
+        u32x4 kr[Tile<D, 64 * kFlatNW>::kPer], vr[Tile<D, 64 * kFlatNW>::kPer];
+        pv_walk<D, kFlatNW, false>(a, a.k + kv, a.v + kv, kr, vr, kb, vb, r.qb, ex, r.lim, r.nfull, static_cast<int>(k.tb),
                             static_cast<int>(k.te), tid, o, lsum);
         lsum += __shfl_xor(lsum, 32);
         if (k.tb == 0 && k.te == k.nt) {
