@@ -167,19 +167,15 @@ __device__ __forceinline__ uint32_t pk_bf16(float a, float b)
 }
 
 // Two exponentials as hi and lo bf16 halves, hi = bf16(e), lo = bf16(e - hi),
-// each pair packed (e0 low, e1 high). e - hi is one v_dot2_f32_bf16 of the
-// packed pair with (-1, 0) or (0, -1), where unpacking and subtracting take
-// two instructions per value; the difference is exact either way.
+// each pair packed (e0 low, e1 high). (e - hi as one v_dot2_f32_bf16 of the
+// packed pair with (-1, 0) or (0, -1) is an instruction a value less, and
+// slower: each needs wait states before its result is packed. 3000 rows of 32
+// heads at D = 64 178.8 us with it, 170.7 so; 1000 after 500 at D = 96 66.8 and
+// 62.8.)
 __device__ __forceinline__ void split2(float e0, float e1, uint32_t &hi, uint32_t &lo)
 {
     hi = pk_bf16(e0, e1);
-    const bf16x2 h = __builtin_bit_cast(bf16x2, hi);
-    // (constants kept in scalar registers: as inline constants of the packed
-    // operand they would not name the half meant)
-    uint32_t c0 = 0x0000BF80u, c1 = 0xBF800000u;
-    asm("" : "+s"(c0), "+s"(c1));
-    lo = pk_bf16(__builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(bf16x2, c0), e0, false),
-                 __builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(bf16x2, c1), e1, false));
+    lo = pk_bf16(e0 - __uint_as_float(hi << 16), e1 - __uint_as_float(hi & 0xFFFF0000u));
 }
 
 // Eight exponentials as hi and lo bf16 halves, packed in k order.
