@@ -98,40 +98,28 @@ __device__ __forceinline__ uint32_t cvt_out(float x)
     return e == 0 ? ((b >> 16) & 0x8000u) : r;
 }
 
-// One row's exponential: see exp_score. From x's exponent t = x c + b.
+// One row's exponential, see exp_score: x's exponent is t = (x - X) c + b.
 struct RowExp {
-    float c, b;
-    // The exponential of x - X where X has the exponent X xc (xc = c, or the
-    // scaled maximum's own factor). Where the exponent of the maximum itself
-    // would leave the f32 range, two scores that differ at all differ by far
-    // more than the exponential's clamp, and a smaller c tells them apart as
-    // well.
-    __device__ __forceinline__ RowExp(float cc, float X, float xc)
-    {
-        c = cc;
-        float t = X * xc;
-        if (__builtin_fabsf(t) > 1e38f) {
-            c *= 0x1p-24f;
-            t = X * (xc * 0x1p-24f);
-        }
-        b = 0.5f - t;
-    }
+    float X, c, b;
     // of scaled scores, m their maximum
-    __device__ __forceinline__ explicit RowExp(float m) : RowExp(1.442695f, m, 1.442695f) {}
+    static __device__ __forceinline__ RowExp scaled(float m) { return RowExp{m, 1.442695f, 0.5f}; }
 };
 
-// P(x - M) of the score x (acc: x or its dot product): t = (x - M) log2(e) + 1/2
-// in one rounding, clamped as the emitted exponential clamps (a NaN too), k =
-// floor(t), and the emitted polynomial about t - k - 1/2, its argument moved
-// by 1/2 into the coefficients: P(x) 2^k = Q(t - k) 2^k. Nine instructions
-// where subtract, clamp, scale, round, subtract, convert, polynomial and
-// ldexp take eleven (and one more for a scale that is no power of two): the
-// causal passes are VALU-bound up to D = 128. Against 64-bit exponentials over
-// |score - M| up to 30, relative rms 1.42e-5 and largest 6.1e-5, both the
+// P(x - M) of the score x (acc: x or its dot product): t = (x - M) log2(e) + 1/2,
+// clamped as the emitted exponential clamps (a NaN too), k = floor(t), and the
+// emitted polynomial about t - k - 1/2, its argument moved by 1/2 into the
+// coefficients: P(x) 2^k = Q(t - k) 2^k. Ten instructions where subtract,
+// clamp, scale, round, subtract, convert, polynomial and ldexp take eleven (and
+// one more for a scale that is no power of two): the causal passes are
+// VALU-bound up to D = 128. The difference is taken first, so that it is exact
+// near the maximum and zero at it, whatever the scores' size; as one fused step
+// x c + (1/2 - M c) the exponent is off by the rounding of M c, which leaves
+// the exponential's range once scores pass 1e9. Against 64-bit exponentials
+// over |score - M| up to 30, relative rms 1.42e-5 and largest 6.1e-5, both the
 // polynomial's own and the same either way.
 __device__ __forceinline__ float exp_score(float acc, const RowExp &x)
 {
-    const float t = __builtin_fmaxf(__builtin_fmaf(acc, x.c, x.b), -125.49977f);
+    const float t = __builtin_fmaxf(__builtin_fmaf(acc - x.X, x.c, x.b), -125.49977f);
     int k;
     asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(k) : "v"(t));
     const float f = __builtin_amdgcn_fractf(t);
@@ -1330,15 +1318,13 @@ __global__ __launch_bounds__(512, 1) void decode_pv_groups(DecodeArgs a)
         if (u == T - 1) smax[cz][ch] = m;
     }
     lds_barrier();
-    // this lane's columns: exponential, last visible key (from j0; a run is at
+    // this lane's columns: maximum, last visible key (from j0; a run is at
     // most 2^30 keys)
-    float ec[NE], eb[NE], lsum[NE];
+    float em[NE], lsum[NE];
     int lim[NE];
 #pragma unroll
     for (int i = 0; i < NE; i++) {
-        const RowExp x(smax[zb + i][j]);
-        ec[i] = x.c;
-        eb[i] = x.b;
+        em[i] = smax[zb + i][j];
         lsum[i] = 0.0f;
         const int64_t last = static_cast<int64_t>(a.past) + ((zb + i) * a.g + j) / a.G - static_cast<int64_t>(j0);
         lim[i] = static_cast<int>(last < -1 ? -1 : last > (1 << 30) ? 1 << 30 : last);
@@ -1351,10 +1337,7 @@ __global__ __launch_bounds__(512, 1) void decode_pv_groups(DecodeArgs a)
         const int i = e / KE, k = e % KE;
         // keys 0 .. vis of the lane's
         const int vis = there ? lim[i] - (static_cast<int>(c0 - j0) + kKeyTile * wt + 8 * G + kb) : -1;
-        RowExp x(0.0f);
-        x.c = ec[i];
-        x.b = eb[i];
-        const float y = exp_score(sc[i][k / 4][k % 4], x);
+        const float y = exp_score(sc[i][k / 4][k % 4], RowExp::scaled(em[i]));
         ev[k & 1] = k <= vis ? y : 0.0f;
         lsum[i] += ev[k & 1];
         if (k & 1) split2(ev[0], ev[1], ph[i][k >> 1], pl[i][k >> 1]);
@@ -1812,8 +1795,8 @@ __global__ __launch_bounds__(512) void decode_combine(DecodeArgs a)
 // The kernels keep the unscaled dot products: q takes the scale's sign as it
 // is loaded (q_sign; |scale| below), so the row maximum of fl(dot * |scale|)
 // is fl(Mraw * |scale|), the rounding being monotonic. An exponential then
-// takes one fused step from the dot product to the exponent, t = dot * c + b
-// with c = |scale| log2(e) and b = 1/2 - Mraw c.
+// takes two steps from the dot product to the exponent, t = (dot - Mraw) c + b
+// with c = |scale| log2(e) and b = 1/2.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ uint32_t q_sign(const PrefillArgs &a) { return a.scale < 0.0f ? 0x80008000u : 0u; }
 __device__ __forceinline__ u32x4 q_chunk(u32x4 v, bool valid, uint32_t sign)
@@ -1823,13 +1806,22 @@ __device__ __forceinline__ u32x4 q_chunk(u32x4 v, bool valid, uint32_t sign)
 
 // A causal row's exponential: m its maximum dot product; with the sink, ms
 // receives the scaled maximum, the larger of the scores' and the sink (vmaxss,
-// decode.rs:239-290).
+// decode.rs:239-290); a sink above the scores moves b by their distance. A scale so
+// small that two dot products may be more than the f32 range apart and their
+// scores still close takes the products by c first (M c is then below 2^9); one
+// whose c would pass the range keeps the scale, where any two scores that
+// differ are further apart than the clamp.
 __device__ __forceinline__ RowExp causal_exp(const PrefillArgs &a, float m, bool sink, float &ms)
 {
-    const float s = __builtin_fabsf(a.scale), c = s * 1.442695f, sm = m * s;
+    const float s = __builtin_fabsf(a.scale), sm = m * s;
     const bool over = sink && !(sm > a.sink);
     ms = over ? a.sink : sm;
-    return RowExp(c, over ? a.sink : m, over ? 1.442695f : c);
+    RowExp x{m, s >= 0x1p127f ? s : s * 1.442695f, over ? __builtin_fmaf(sm - a.sink, 1.442695f, 0.5f) : 0.5f};
+    if (s < 0x1p-120f) {
+        x.X = 0.0f;
+        x.b -= m * x.c;
+    }
+    return x;
 }
 
 // A row's normalisation: the division by its sum, or (the sink) the
