@@ -387,9 +387,9 @@ DecodeCfg decode_cfg(const hsdpa_plan *p, uint64_t rows, uint64_t n, int sub, bo
                         ? hsdpa::kDecodeKeysPV
                         : static_cast<int>(run);
     }
-    // D = 256, past one round of 256-key workgroups per group: pass 2 takes all
-    // the groups of a KV head in each workgroup, in one round of runs of whole
-    // tiles (decode_pv_groups_ok)
+    // D = 128 and 256, past one round of 256-key workgroups per group: pass 2
+    // takes all the groups of a KV head in each workgroup, in one round of runs
+    // of whole tiles (decode_pv_groups_ok)
     if (!fused && groups * nch > cu1) {
         // (a narrow workspace may hold fewer)
         const uint64_t wgs = hsdpa::decode_pv_groups_wgs(p->kv_heads, cu1);
@@ -619,7 +619,7 @@ static hsdpa_status run_part(const hsdpa_plan *plan, const hsdpa_call *call, con
             plan->dec_part)
             return HSDPA_ERR_WORKSPACE;
         if (kernels) *kernels = rows == 1 ? HSDPA_KERNELS_DECODE : HSDPA_KERNELS_FEW_ROWS;
-        if (splits) *splits = 1;
+        if (splits) *splits = c.pv_all && !c.direct ? 0 : 1;
         if (launches) *launches += c.direct ? 2 : 3;
         if (!launch) return HSDPA_OK;
         hsdpa::DecodeArgs a{};
@@ -709,15 +709,15 @@ static hsdpa_status run_part(const hsdpa_plan *plan, const hsdpa_call *call, con
     }
     const int sp = hsdpa::prefill_split_count(a, d, static_cast<int>(s.heads), ps);
     const bool paired = sp == 1 && hsdpa::prefill_pair_rows(a, d, static_cast<int>(s.heads), ps).srows > 0;
-    // the equal shares are a split over the keys, or (where pairs of row groups
-    // would do) those row groups evened out further
+    // the equal shares (splits 0) go by the form whose place they take: a split
+    // over the keys, or pairs of row groups evened out further
     hsdpa::FlatShape flat_shape;
     const bool flat = hsdpa::prefill_flat_shape(a, d, static_cast<int>(s.heads), ps, flat_shape);
     if (kernels)
         *kernels = paired ? HSDPA_KERNELS_CAUSAL_PAIRED
                    : sp > 1 || flat ? HSDPA_KERNELS_CAUSAL_SPLIT
                                     : HSDPA_KERNELS_CAUSAL;
-    if (splits) *splits = static_cast<uint32_t>(flat && !paired && sp == 1 ? 2 : sp);
+    if (splits) *splits = flat ? 0u : static_cast<uint32_t>(sp);
     if (launches) *launches += sp > 1 || paired || flat ? 3 : 1;
     if (!launch) return HSDPA_OK;
     const hipError_t e = hsdpa::launch_prefill(a, d, static_cast<int>(s.heads), ps, st);

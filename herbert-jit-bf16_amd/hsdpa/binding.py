@@ -192,7 +192,9 @@ class Plan:
         return int(library().hsdpa_workspace_bytes(self._h))
 
     def route(self, rows: int, past: int) -> dict:
-        """The kernels a call of `rows` rows after `past` positions would run."""
+        """The kernels a call of `rows` rows after `past` positions would run
+        (splits: key splits of causal_split, 0 for causal calls in equal shares and
+        for decode passes over all groups, else 1)."""
         r = Route()
         rc = library().hsdpa_attention_route(self._h, rows, past, ctypes.byref(r))
         if rc != 0:

@@ -187,7 +187,9 @@ typedef struct hsdpa_route {
     uint32_t tail;          /* hsdpa_kernels of the last tail_rows rows (NONE: no tail) */
     uint32_t tail_form;
     uint64_t main_rows, tail_rows;
-    uint32_t splits;        /* key splits of CAUSAL_SPLIT, else 1 */
+    uint32_t splits;        /* key splits of CAUSAL_SPLIT, else 1; 0 where the workgroups share the work
+                               otherwise: CAUSAL_SPLIT or CAUSAL_PAIRED in equal shares, DECODE or
+                               FEW_ROWS with pass 2 over all the groups of a KV head per workgroup */
     uint32_t launches;      /* kernel launches of the whole call */
 } hsdpa_route;
 

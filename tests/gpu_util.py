@@ -19,3 +19,10 @@ def run_hsdpa(w, plan=None, stream=None) -> np.ndarray:
     hsdpa.attention_torch(plan, q, k, v, out, w.rows, w.past, w.scale, ws, stream)
     torch.cuda.synchronize()
     return out.cpu().numpy().view(np.uint16)
+
+
+def cus() -> int:
+    """Compute units of the current GPU, which the kernels' grids follow."""
+    import torch
+
+    return torch.cuda.get_device_properties(torch.cuda.current_device()).multi_processor_count
