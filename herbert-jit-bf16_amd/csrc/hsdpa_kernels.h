@@ -412,18 +412,20 @@ struct FlatShape {
 // Workspace for them: cells of 8 waves x 32 rows, two a workgroup.
 constexpr int kFlatDim = 128;
 inline uint64_t prefill_flat_units(int d, uint64_t units) { return d == kFlatDim ? 2 * units : units; }
-// Whether the equal shares take a call whose grid's longest workgroup walks
-// `longest` tiles (0: more than one round of them; row group by row group, in
-// pairs or split): where a share, with three tiles for its second row group's
-// start, is an eighth shorter, the longest row group sees more than
-// kFlatMinLongest tiles (as for kPairMinLongest, fewer than which do not pay
-// two more launches), and the workspace holds the parts. 1800 rows of 32/8
-// heads with no cache 131.4 -> 117.6 us, 700 after 900 with the sink 78.4 ->
-// 68.4; calls that fill their round already stay as they were.
+// Whether the equal shares take a call that the form it would take otherwise
+// does in `other` quarters of a key tile's time (0: more than one round of its
+// workgroups): where they take fewer, the longest row group sees more than
+// kFlatMinLongest tiles (fewer do not pay two more launches), and the workspace
+// holds the parts. A share takes its tiles, four tiles for each (head group, row
+// group) piece it has (Q, the first tiles, the piece's maxima and outputs), and
+// a quarter for each of a row group's maxima, which P.V reads in turn: a call
+// within 3.5 % of 25 + 1.96 (tiles + 4 pieces) us over 650 calls. With no cache
+// the first row groups are short and a share holds many: 3 238 rows of 16/2
+// heads 9 pieces, 193 us, paired 147; 2 122 after 5 515 274 us, 452 as one round.
 constexpr uint64_t kFlatMinLongest = 40;
-inline bool prefill_flat(const PrefillArgs &a, int d, int heads, const PrefillSplit &ps, uint64_t longest, FlatShape &f)
+inline bool prefill_flat(const PrefillArgs &a, int d, int heads, const PrefillSplit &ps, uint64_t other, FlatShape &f)
 {
-    if (d != kFlatDim || longest == 0 || ps.cus <= 0) return false;
+    if (d != kFlatDim || other == 0 || ps.cus <= 0) return false;
     const uint64_t cus = static_cast<uint64_t>(ps.cus), h = static_cast<uint64_t>(heads);
     f.lh = a.gqa % 8 == 0 ? 3 : a.gqa % 4 == 0 ? 2 : a.gqa % 2 == 0 ? 1 : 0;
     const uint64_t RB = 8u >> f.lh, R = (a.rows + 32 * RB - 1) / (32 * RB);
@@ -431,9 +433,20 @@ inline bool prefill_flat(const PrefillArgs &a, int d, int heads, const PrefillSp
     if (last <= kFlatMinLongest || last > (1u << 20) || R > (1u << 12)) return false;
     const uint64_t Th = (R - 1) * p0 + RB * ((R - 1) * R / 2) + last, T = Th * (h >> f.lh);
     const uint64_t wp = cus, wm = 2 * cus;                      // the maxima's registers allow two per unit
-    if ((T + 1) * wm > 0xFFFFFFFFull || T < 4 * wm || 8 * (T / cus + 3) > 7 * longest) return false;
+    if ((T + 1) * wm > 0xFFFFFFFFull || T < 4 * wm || 4 * T / cus >= other) return false;
     if (a.rows * h > 0x7FFFFFFFull || 16 * wp > ps.flat_units) return false;
-    if ((last / (T / wm) + 2) * h * a.rows > ps.flat_units * kSplitMaxCells) return false;
+    const uint64_t slots = last / (T / wm) + 2;
+    if (slots * h * a.rows > ps.flat_units * kSplitMaxCells) return false;
+    // the most pieces of a share: two where it ends inside one row group and
+    // starts the next, more where it starts a head group's short ones
+    uint64_t pieces = 2;
+    for (uint64_t s = 0; s < T; s += Th) {
+        const uint64_t w = ((s + 1) * wp - 1) / T, x0 = w * T / wp, len = (w + 1) * T / wp - s;
+        uint64_t n = x0 < s ? 1 : 0;
+        for (uint64_t r = 0; r < R && r * p0 + RB * (r * (r + 1) / 2) < len; r++) n++;
+        if (n > pieces) pieces = n;
+    }
+    if (4 * T / cus + 16 * pieces + slots >= other) return false;
     f.smax = ps.smax;
     f.so = ps.so;
     f.sl = ps.sl;

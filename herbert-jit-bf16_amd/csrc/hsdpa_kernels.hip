@@ -402,14 +402,25 @@ PairRows prefill_pair_rows(const PrefillArgs &a, int head_dim, int heads, const 
 
 bool prefill_flat_shape(const PrefillArgs &a, int head_dim, int heads, const PrefillSplit &ps, FlatShape &f)
 {
-    if (head_dim != kFlatDim || ps.flat_units == 0) return false;
-    const dim3 g = prefill_grid(a, head_dim, heads);
     const uint64_t tiles = (a.past + a.rows + kKeyTile - 1) / kKeyTile;
+    if (head_dim != kFlatDim || ps.flat_units == 0 || tiles <= kFlatMinLongest) return false;
+    const dim3 g = prefill_grid(a, head_dim, heads);
     const uint64_t splits = static_cast<uint64_t>(prefill_split_count(a, head_dim, heads, ps));
     const PairRows pr = prefill_pair_rows(a, head_dim, heads, ps);
     const bool one_round = static_cast<uint64_t>(g.x) * g.y <= static_cast<uint64_t>(ps.cus);
-    const uint64_t longest = splits > 1 ? (tiles + splits - 1) / splits : pr.srows ? pr.longest : one_round ? tiles : 0;
-    return prefill_flat(a, head_dim, heads, ps, longest, f);
+    // the form it would take otherwise, in quarters of a tile's time (1.96 us a
+    // tile): an even split, pairs (their maxima run two workgroups per unit, their
+    // partials' bytes count) or one launch. The constants, what the form's
+    // launches take more or less than the equal shares' (prefill_flat), and with
+    // the sink that its kernels stage K and V for each head: fitted to 650 calls
+    // timed both ways and shifted so that neither side loses much, on 300 other
+    // calls at most 6 % against the better one
+    const uint64_t other =
+        splits > 1 ? 4 * ((tiles + splits - 1) / splits) + (a.sink_on ? 20 : 9)
+        : pr.srows ? 17 * pr.longest / 5 + 12 * a.rows * static_cast<uint64_t>(heads) / 10000 + 4
+        : one_round ? 4 * tiles - 27 + 24 / static_cast<uint64_t>(prefill_hpw(a, head_dim))
+                    : 0;
+    return prefill_flat(a, head_dim, heads, ps, other, f);
 }
 
 template <int D, int HPW>
