@@ -383,20 +383,26 @@ DecodeCfg decode_cfg(const hsdpa_plan *p, uint64_t rows, uint64_t n, int sub, bo
         const uint64_t tiles = (n + hsdpa::kKeyTile - 1) / hsdpa::kKeyTile;
         const uint64_t run = hsdpa::kKeyTile * ((tiles + per - 1) / per);
         c.keys_pv = groups * nch <= cu1 || !hsdpa::decode_pv_loop_ok(d, c.g, static_cast<int>(rows), fused) ||
+                            !hsdpa::decode_pv_loop_rows_ok(d, static_cast<int>(rows), sub, p->kv_heads * nch, cu1) ||
                             run > (1u << 30)
                         ? hsdpa::kDecodeKeysPV
                         : static_cast<int>(run);
     }
     // D = 128 and 256, past one round of 256-key workgroups per group: pass 2
-    // takes all the groups of a KV head in each workgroup, in one round of runs
-    // of whole tiles (decode_pv_groups_ok)
+    // may take all the groups of a KV head in each workgroup, in one round of
+    // runs of whole tiles, where that is shorter than the form chosen above
+    // (decode_pv_groups_ok, decode_pv_groups_shorter)
     if (!fused && groups * nch > cu1) {
-        // (a narrow workspace may hold fewer)
+        // (a narrow workspace, or a short cache's, may hold fewer)
         const uint64_t wgs = hsdpa::decode_pv_groups_wgs(p->kv_heads, cu1);
-        const uint64_t per = std::min(wgs, p->dec_part / (static_cast<uint64_t>(sub) * static_cast<uint64_t>(c.g)));
+        const uint64_t cols_wg = static_cast<uint64_t>(sub) * static_cast<uint64_t>(c.g);
+        const uint64_t per = std::min(wgs, p->dec_part / cols_wg);
         const uint64_t tiles = (n + hsdpa::kKeyTile - 1) / hsdpa::kKeyTile;
         const uint64_t run = per ? std::max<uint64_t>((tiles + per - 1) / per, 4) : 0;
-        if (2 * per >= wgs && hsdpa::decode_pv_groups_ok(d, sub, c.g, run)) {
+        const uint64_t other = (n + c.keys_pv - 1) / c.keys_pv;  // that form's workgroups per group
+        if (run && hsdpa::decode_pv_groups_ok(d, sub, c.g, run) &&
+            (hsdpa::decode_pv_groups_shorter(d, sub, run, groups, other, c.keys_pv, cu1) ||
+             other * cols_wg > p->dec_part)) {
             c.keys_pv = static_cast<int>(run) * hsdpa::kKeyTile;
             c.pv_all = 1;
         }

@@ -258,35 +258,57 @@ inline bool decode_direct_ok(int d, int rows, int sub, int g, uint64_t n, bool f
 // the tuned head dimensions; under the Fused form at D = 256 for one row in
 // groups of up to 8 columns (with 16 its running maxima and corrections and
 // the P columns' operands no longer fit beside the next chunk's V tile), under
-// the Chained form where decode_pv_groups does not take the call.
+// the Chained form where decode_pv_groups does not take the call
+// (decode_pv_loop_rows_ok).
 inline bool decode_pv_loop_ok(int d, int g, int rows, bool fused)
 {
     return d == 64 || d == 128 || (d == 256 && (!fused || (g <= 8 && rows == 1)));
+}
+// Several rows at D = 256 in 2 or more groups: runs per group stream V once for
+// each group in one round of workgroups; with more than 4 groups, or where the
+// cache is one round of 256-key workgroups for the KV heads alone, those (the
+// groups of a key range on one XCD, whose L2 serves V to the later ones) were
+// faster: 16 rows of 16 heads on 2 KV heads after 64K 131.4 us in runs, 126.6.
+inline bool decode_pv_loop_rows_ok(int d, int rows, int sub, uint64_t kv_chunks, uint64_t cus)
+{
+    return d != 256 || rows == 1 || sub == 1 || (sub <= 4 && kv_chunks > cus);
 }
 // Pass 2 over every group of a KV head in one workgroup (decode_pv_groups),
 // past one round of 256-key workgroups per group (below, the groups'
 // exponentials run beside each other on compute units that would idle: 8 rows
 // of 8 heads on 2 KV heads after 1000 and 8184 keys 14.6 and 20.5 us, 17.0 and
-// 23.8 this way). Past it, us a call by a group or a round of 256-key
-// workgroups at a time and this way: 8 rows after 8 192 27.8 -> 26.0, 32 768
-// 57.6 -> 41.0, 131 000 116 -> 90; 4 rows after 32 764 30.9 -> 28.8, 65 536
-// 54 -> 45; 16 rows after 32 752 58.7 -> 54.0; 2 rows (one group of 16
-// columns) after 32 768 29.6 -> 26.5; 32 heads per KV head at 33 000 40 ->
-// 33. One group of at most 8 columns takes it only where the run of tiles
-// leaves the 256-key chunks of decode_pv one or two tiles over (`run` whole
-// tiles a workgroup), which costs those a whole chunk: one row at 32 769 and
-// 40 001 25.4 and 27.0 -> 24.5 and 26.4, but 49 153 and 131 072 (12 and 32
-// tiles) 29.7 and 55.9 -> 31.3 and 58.4. At D = 128 (chunks of 8 tiles) from
-// runs of 6 tiles on: 8 rows of 8 heads on 4 KV heads after 8 000 (4 tiles)
-// 23.7 us and 26.0 this way, after 16 000, 32 000 and 131 000 31.4, 51.5 and
-// 154 -> 28.6, 42.5 and 105. Runs past 2^25 tiles (2^30 keys) are
-// left to decode_pv.
+// 23.8 this way), in runs of `run` whole tiles, at D = 128 (chunks of 8 tiles)
+// of 6 at least. One group of at most 8 columns takes it only where the run
+// leaves the 256-key chunks of decode_pv one or two tiles over, which costs those a
+// whole chunk: one row at 32 769 and 40 001 25.4 and 27.0 -> 24.5 and 26.4,
+// but 49 153 and 131 072 (12 and 32 tiles) 29.7 and 55.9 -> 31.3 and 58.4. Runs
+// past 2^25 tiles (2^30 keys) are left to decode_pv.
 inline bool decode_pv_groups_dim(int d, int sub) { return (d == 128 || d == 256) && sub >= 1 && sub <= kDecodeMaxSub; }
+inline bool decode_pv_groups_rest(int d, int sub, int g, uint64_t run)
+{
+    return d == 256 && sub == 1 && g <= 8 && (run % 8 == 1 || run % 8 == 2) && run < 32;
+}
 inline bool decode_pv_groups_ok(int d, int sub, int g, uint64_t run)
 {
-    const bool rest = run % 8 == 1 || run % 8 == 2;
     return decode_pv_groups_dim(d, sub) && run <= (uint64_t{1} << 25) && (d == 256 || run >= 6) &&
-           (sub > 1 || g > 8 || (d == 256 && rest && run < 32));
+           (sub > 1 || g > 8 || decode_pv_groups_rest(d, sub, g, run));
+}
+// Whether such runs are shorter than decode_pv's way, nwg workgroups of keys_pv
+// keys for each of `groups` groups: tiles times groups in turn on the busiest
+// compute unit, decode_pv's in whole 256-key chunks and (several groups) with a
+// key range's workgroups on one of 8 XCDs. Per tile and group it is the faster
+// by about a fifth, except that a chunk of D = 128 costs a whole one. 240
+// calls of 2 to 16 rows timed both ways: 1.21x where it says so, 0.94 at worst;
+// 14 rows of 8 heads on 2 KV heads after 7 982 keys (28 against 16) 33.6 us, 28.7
+// the other way, after 27 312 (49 against 64) 48.1 and 66.0; at D = 128 16
+// rows of 4 heads on 8 after 5 147 (32 against 24) 31.0 and 29.8, 6 of 8 on 16
+// after 6 130 (36 against 128) 37.0 and 51.5.
+inline bool decode_pv_groups_shorter(int d, int sub, uint64_t run, uint64_t groups, uint64_t nwg, int keys_pv, uint64_t cus)
+{
+    const uint64_t xcu = cus / 8 > 0 ? cus / 8 : 1, chunk = 8;
+    const uint64_t rounds = sub > 1 ? ((nwg + 7) / 8 * groups + xcu - 1) / xcu : (nwg * groups + cus - 1) / cus;
+    const uint64_t other = rounds * chunk * ((static_cast<uint64_t>(keys_pv) + kDecodeKeysPV - 1) / kDecodeKeysPV);
+    return 5 * static_cast<uint64_t>(sub) * (d == 128 && run < chunk ? chunk : run) <= 6 * other;
 }
 // Its workgroups per KV head: one round of the compute units.
 inline uint64_t decode_pv_groups_wgs(uint64_t kv_heads, uint64_t cus) { return cus > kv_heads ? cus / kv_heads : 1; }

@@ -12,7 +12,7 @@ import oracle
 from hsdpa import workloads as W
 from parity import assert_parity
 
-from gpu_util import run_hsdpa
+from gpu_util import cus, run_hsdpa
 
 pytestmark = pytest.mark.gpu
 
@@ -57,6 +57,8 @@ def test_groups_parity(torch_cuda, case):
     w = W.make(name, heads=h, kv_heads=kvh, head_dim=dim, rows=rows, past=past, seed=91)
     plan = hsdpa.Plan(w.heads, w.gqa, w.head_dim, w.capacity, sink=sink is not None)
     print(f"case {name}", flush=True)
+    if cus() == 256:                # the shapes are chosen for 256 compute units
+        assert plan.route(rows, past)["splits"] == 0, "not over all groups"
     if sink is None:
         out, ref = run_hsdpa(w, plan), oracle.attention(w)
     else:
@@ -67,3 +69,26 @@ def test_groups_parity(torch_cuda, case):
         torch.cuda.synchronize()
         out, ref = o.cpu().numpy().view(np.uint16), oracle.attention(w, sink=sink)
     assert_parity(out, ref, w, name)
+
+
+# plans whose workspace holds fewer workgroups, at rows and lengths where that
+# decides the form (name, heads, kv_heads, head_dim, rows, past, capacity, max_rows, over all groups)
+SMALLER = [
+    ("static_16_rows", 16, 2, 256, 16, 6000, 12000, 16, False),
+    ("static_12_rows_full", 16, 2, 256, 12, 11988, 12000, 16, False),
+    ("static_8_rows", 16, 2, 256, 8, 11900, 12000, 16, True),
+    ("short_cache_11_rows", 128, 16, 256, 11, 610, 621, 11, True),
+    ("static_d128_8_rows", 32, 4, 128, 8, 29000, 30000, 8, False),
+]
+
+
+@pytest.mark.parametrize("case", SMALLER, ids=[c[0] for c in SMALLER])
+def test_smaller_workspaces(torch_cuda, case):
+    name, h, kvh, dim, rows, past, cap, max_rows, groups = case
+    w = W.make(name, heads=h, kv_heads=kvh, head_dim=dim, rows=rows, past=past, seed=92, capacity=cap)
+    plan = hsdpa.Plan(w.heads, w.gqa, w.head_dim, cap, max_rows=max_rows)
+    print(f"case {name} {plan.route(rows, past)}", flush=True)
+    if cus() == 256:
+        assert plan.workspace_bytes <= 32 << 20
+        assert (plan.route(rows, past)["splits"] == 0) == groups
+    assert_parity(run_hsdpa(w, plan), oracle.attention(w), w, name)
