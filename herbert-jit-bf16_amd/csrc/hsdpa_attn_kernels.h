@@ -1801,7 +1801,7 @@ __global__ __launch_bounds__(512) void decode_combine(DecodeArgs a)
 __device__ __forceinline__ uint32_t q_sign(const PrefillArgs &a) { return a.scale < 0.0f ? 0x80008000u : 0u; }
 __device__ __forceinline__ u32x4 q_chunk(u32x4 v, bool valid, uint32_t sign)
 {
-    return valid ? v ^ sign : u32x4{0, 0, 0, 0};
+    return (v ^ sign) & (valid ? 0xFFFFFFFFu : 0u);             // one v_bitop3 a word
 }
 
 // A causal row's exponential: m its maximum dot product; with the sink, ms
@@ -2058,7 +2058,7 @@ __global__ __launch_bounds__(64 * NW, 1) void prefill_attn(PrefillArgs a)
             // keys t0 + k with k <= vis are visible to this row
             const int vis = static_cast<int>(static_cast<int64_t>(lim) - static_cast<int64_t>(t0));
 #pragma unroll
-            for (int r = 0; r < 16; r++) 
+            for (int r = 0; r < 16; r++)
                 if (key_of(r, grp) <= vis) m = __builtin_fmaxf(m, acc[r]);
         }
         if (!last) tile_lstore_padded<D, THREADS>(kb[(t + 1) & 1], SK, tid, kr);
@@ -2186,7 +2186,7 @@ __global__ __launch_bounds__(64 * KS, 1) void prefill_ks(PrefillArgs a)
                 } else {
                     const int vis = static_cast<int>(static_cast<int64_t>(lim) - static_cast<int64_t>(t0));
 #pragma unroll
-                    for (int r = 0; r < 16; r++) 
+                    for (int r = 0; r < 16; r++)
                         if (key_of(r, grp) <= vis) m = __builtin_fmaxf(m, acc[r]);
                 }
                 wave_sync();
