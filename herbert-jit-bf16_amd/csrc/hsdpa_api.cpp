@@ -529,9 +529,9 @@ static void plan_layout(hsdpa_plan *p, uint64_t cols, bool narrow)
         causal = reaches_causal(p, r);
     p->split_units = causal ? std::min<uint64_t>(hsdpa::kSplitUnits, 8 * static_cast<uint64_t>(p->cus)) : 0;
     // (the equal shares at D = 128: two cells a workgroup)
-    p->flat_units = narrow || cap <= hsdpa::kFlatMinLongest * hsdpa::kKeyTile
-                        ? p->split_units
-                        : hsdpa::prefill_flat_units(static_cast<int>(d), p->split_units);
+    p->flat_units = narrow ? p->split_units
+                           : hsdpa::prefill_flat_units(static_cast<int>(d), g, p->spec.heads, cap, p->max_rows,
+                                                       static_cast<uint64_t>(p->cus), p->split_units);
     const uint64_t cells = p->flat_units * 32;
     p->off_smax = off;
     off = align_up(off + p->flat_units * hsdpa::kSplitMaxCells * 4, kAlign);

@@ -431,9 +431,40 @@ struct FlatShape {
     float *smax, *so, *sl;
     uint32_t T, Th, R, p0, last, lh, heads, wm, wp; // row group rg has p0 + (rg + 1) 8 / HPW tiles, the last `last`
 };
-// Workspace for them: cells of 8 waves x 32 rows, two a workgroup.
 constexpr int kFlatDim = 128;
-inline uint64_t prefill_flat_units(int d, uint64_t units) { return d == kFlatDim ? 2 * units : units; }
+constexpr uint64_t kFlatMinLongest = 40;
+// a call's tiles, one after the other
+struct FlatTiles {
+    uint64_t lh, RB, R, p0, last, Th, T;
+    FlatTiles(uint64_t rows, uint64_t past, uint64_t gqa, uint64_t heads)
+    {
+        lh = gqa % 8 == 0 ? 3 : gqa % 4 == 0 ? 2 : gqa % 2 == 0 ? 1 : 0;
+        RB = 8u >> lh;
+        R = (rows + 32 * RB - 1) / (32 * RB);
+        p0 = (past + kKeyTile - 1) / kKeyTile;
+        last = (past + rows + kKeyTile - 1) / kKeyTile;
+        Th = (R - 1) * p0 + RB * ((R - 1) * R / 2) + last;
+        T = Th * (heads >> lh);
+    }
+};
+// row maxima shares (their registers allow two workgroups per unit), four tiles
+// each at least
+inline uint64_t flat_max_shares(uint64_t cus) { return 2 * cus; }
+inline uint64_t flat_min_tiles(uint64_t cus) { return 4 * flat_max_shares(cus); }
+// Workspace for them: cells of 8 waves x 32 rows, two a workgroup, where a
+// plan's calls can have the tiles for them: at most those of all its positions
+// with `max_rows` of them rows, and RB + 1 a row group more (fewer rows end
+// elsewhere in a tile and a row group). Half as much serves the other forms (8/2
+// heads 35 and 68 MiB).
+inline uint64_t prefill_flat_units(int d, uint64_t gqa, uint64_t heads, uint64_t cap, uint64_t max_rows, uint64_t cus,
+                                   uint64_t units)
+{
+    if (d != kFlatDim || max_rows == 0 || cap > (uint64_t{1} << 26) || heads > (uint64_t{1} << 16))
+        return d == kFlatDim ? 2 * units : units;               // past what the count below holds
+    const FlatTiles t(max_rows, cap - max_rows, gqa, heads);
+    const uint64_t most = t.T + (t.RB + 1) * t.R * (heads >> t.lh);
+    return t.last > kFlatMinLongest && most >= flat_min_tiles(cus) ? 2 * units : units;
+}
 // Whether the equal shares take a call that the form it would take otherwise
 // does in `other` quarters of a key tile's time (0: more than one round of its
 // workgroups): where they take fewer, the longest row group sees more than
@@ -444,18 +475,15 @@ inline uint64_t prefill_flat_units(int d, uint64_t units) { return d == kFlatDim
 // within 3.5 % of 25 + 1.96 (tiles + 4 pieces) us over 650 calls. With no cache
 // the first row groups are short and a share holds many: 3 238 rows of 16/2
 // heads 9 pieces, 193 us, paired 147; 2 122 after 5 515 274 us, 452 as one round.
-constexpr uint64_t kFlatMinLongest = 40;
 inline bool prefill_flat(const PrefillArgs &a, int d, int heads, const PrefillSplit &ps, uint64_t other, FlatShape &f)
 {
     if (d != kFlatDim || other == 0 || ps.cus <= 0) return false;
     const uint64_t cus = static_cast<uint64_t>(ps.cus), h = static_cast<uint64_t>(heads);
-    f.lh = a.gqa % 8 == 0 ? 3 : a.gqa % 4 == 0 ? 2 : a.gqa % 2 == 0 ? 1 : 0;
-    const uint64_t RB = 8u >> f.lh, R = (a.rows + 32 * RB - 1) / (32 * RB);
-    const uint64_t p0 = (a.past + kKeyTile - 1) / kKeyTile, last = (a.past + a.rows + kKeyTile - 1) / kKeyTile;
+    const FlatTiles t(a.rows, a.past, static_cast<uint64_t>(a.gqa), h);
+    const uint64_t RB = t.RB, R = t.R, p0 = t.p0, last = t.last, Th = t.Th, T = t.T;
     if (last <= kFlatMinLongest || last > (1u << 20) || R > (1u << 12)) return false;
-    const uint64_t Th = (R - 1) * p0 + RB * ((R - 1) * R / 2) + last, T = Th * (h >> f.lh);
-    const uint64_t wp = cus, wm = 2 * cus;                      // the maxima's registers allow two per unit
-    if ((T + 1) * wm > 0xFFFFFFFFull || T < 4 * wm || 4 * T / cus >= other) return false;
+    const uint64_t wp = cus, wm = flat_max_shares(cus);
+    if ((T + 1) * wm > 0xFFFFFFFFull || T < flat_min_tiles(cus) || 4 * T / cus >= other) return false;
     if (a.rows * h > 0x7FFFFFFFull || 16 * wp > ps.flat_units) return false;
     const uint64_t slots = last / (T / wm) + 2;
     if (slots * h * a.rows > ps.flat_units * kSplitMaxCells) return false;
@@ -469,6 +497,7 @@ inline bool prefill_flat(const PrefillArgs &a, int d, int heads, const PrefillSp
         if (n > pieces) pieces = n;
     }
     if (4 * T / cus + 16 * pieces + slots >= other) return false;
+    f.lh = static_cast<uint32_t>(t.lh);
     f.smax = ps.smax;
     f.so = ps.so;
     f.sl = ps.sl;
