@@ -29,6 +29,7 @@ CASES = [
     ("split_64", 8, 2, 64, 300, 1500, False, "causal_split"),
     ("split_256_sink", 4, 1, 256, 64, 900, True, "causal_split"),
     ("paired_64", 16, 2, 64, 2200, 0, False, "causal_paired"),
+    ("paired_64_sink", 16, 2, 64, 2200, 0, True, "causal_paired"),
     ("shares_128", 32, 8, 128, 1300, 0, False, None),
     ("shares_128_sink", 32, 4, 128, 700, 905, True, None),
     ("groups_256", 128, 16, 256, 4, 2300, False, "few_rows"),
