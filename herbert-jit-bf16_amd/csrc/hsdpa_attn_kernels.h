@@ -1816,7 +1816,11 @@ __device__ __forceinline__ RowExp causal_exp(const PrefillArgs &a, float m, bool
     const float s = __builtin_fabsf(a.scale), sm = m * s;
     const bool over = sink && !(sm > a.sink);
     ms = over ? a.sink : sm;
-    RowExp x{m, s >= 0x1p127f ? s : s * 1.442695f, over ? __builtin_fmaf(sm - a.sink, 1.442695f, 0.5f) : 0.5f};
+    // c in a scalar register: one vector register more, and the short chunk's
+    // kernel of 32 tiles at D = 128 runs one wave per SIMD instead of two
+    const float c = __uint_as_float(
+        __builtin_amdgcn_readfirstlane(__float_as_uint(s >= 0x1p127f ? s : s * 1.442695f)));
+    RowExp x{m, c, over ? __builtin_fmaf(sm - a.sink, 1.442695f, 0.5f) : 0.5f};
     if (s < 0x1p-120f) {
         x.X = 0.0f;
         x.b -= m * x.c;
