@@ -115,8 +115,9 @@ struct RowExp {
 // near the maximum and zero at it, whatever the scores' size; as one fused step
 // x c + (1/2 - M c) the exponent is off by the rounding of M c, which leaves
 // the exponential's range once scores pass 1e9. Against 64-bit exponentials
-// over |score - M| up to 30, relative rms 1.42e-5 and largest 6.1e-5, both the
-// polynomial's own and the same either way.
+// of the same scores, |score - M| up to 30: relative rms 1.4e-5 and largest
+// 6.3e-5, the polynomial's own; the emitted sequence the same where the scale is a
+// power of two or M small, 2.9e-4 and 6.0e-4 where it rounds scores of 1e4.
 __device__ __forceinline__ float exp_score(float acc, const RowExp &x)
 {
     const float t = __builtin_fmaxf(__builtin_fmaf(acc - x.X, x.c, x.b), -125.49977f);
@@ -1215,8 +1216,8 @@ __global__ __launch_bounds__(64 * W, D > 256 ? 1 : 8 / W) void decode_pv(DecodeA
 // Bound by its phases' latency over short runs and by the stream over long
 // ones. Before (a group at a time, its P columns through LDS element by
 // element, two barriers each): 21.8 us of a call for 8 rows of 8 heads on 2 KV
-// heads after 32 760 keys and 36.5 after 32 768, now 14.4 and 16.1; whole calls
-// at decode_pv_groups_ok.
+// heads after 32 760 keys and 36.5 after 32 768, now 18.0 and 19.2 (kernel
+// trace); whole calls at decode_pv_groups_shorter.
 // The partials go where decode_pv puts them. Each column carries its row's
 // causal limit.
 // ---------------------------------------------------------------------------

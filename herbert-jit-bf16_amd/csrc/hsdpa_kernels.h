@@ -298,7 +298,8 @@ inline bool decode_pv_groups_ok(int d, int sub, int g, uint64_t run)
 // compute unit, decode_pv's in whole 256-key chunks and (several groups) with a
 // key range's workgroups on one of 8 XCDs. Per tile and group it is the faster
 // by about a fifth, except that a chunk of D = 128 costs a whole one. 240
-// calls of 2 to 16 rows timed both ways: 1.21x where it says so, 0.94 at worst;
+// calls of 2 to 16 rows timed both ways: 1.16x over the 178 where it says so, 0.94
+// at worst;
 // 14 rows of 8 heads on 2 KV heads after 7 982 keys (28 against 16) 33.6 us, 28.7
 // the other way, after 27 312 (49 against 64) 48.1 and 66.0; at D = 128 16
 // rows of 4 heads on 8 after 5 147 (32 against 24) 31.0 and 29.8, 6 of 8 on 16
@@ -474,7 +475,8 @@ inline uint64_t prefill_flat_units(int d, uint64_t gqa, uint64_t heads, uint64_t
 // a quarter for each of a row group's maxima, which P.V reads in turn: a call
 // within 3.5 % of 25 + 1.96 (tiles + 4 pieces) us over 650 calls. With no cache
 // the first row groups are short and a share holds many: 3 238 rows of 16/2
-// heads 9 pieces, 193 us, paired 147; 2 122 after 5 515 274 us, 452 as one round.
+// heads 9 pieces, 193 us, paired 147; 2 122 after 5 515 274 us, 452 as one round;
+// 1 800 of 32/8 heads 123.5, 145.8; 700 after 900 with the sink 69.9, 83.5.
 inline bool prefill_flat(const PrefillArgs &a, int d, int heads, const PrefillSplit &ps, uint64_t other, FlatShape &f)
 {
     if (d != kFlatDim || other == 0 || ps.cus <= 0) return false;

@@ -10,8 +10,8 @@
 // arguments here, so that there is one instantiation. At D = 256 the grids that
 // start every workgroup at tile 0 stay: a KV head does not fit an XCD's L2,
 // which then serves the workgroups that walk the same tiles at the same time.
-// At the smaller head dimensions the shares' parts would take plans past the
-// static scratch that fit it.
+// The smaller head dimensions have no instantiation and are not measured this
+// way; a plan whose static scratch the parts would pass is laid out without them.
 
 #include "hsdpa_attn_kernels.h"
 
