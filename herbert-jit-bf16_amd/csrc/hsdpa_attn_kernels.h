@@ -1807,7 +1807,9 @@ __device__ __forceinline__ u32x4 q_chunk(u32x4 v, bool valid, uint32_t sign)
 
 // A causal row's exponential: m its maximum dot product; with the sink, ms
 // receives the scaled maximum, the larger of the scores' and the sink (vmaxss,
-// decode.rs:239-290); a sink above the scores moves b by their distance. A scale so
+// decode.rs:239-290); a sink above the scores moves b by their distance. A scaled
+// maximum past the f32 range makes b a NaN: every weight is then the clamp's, as
+// the emitted sequence gives it. A scale so
 // small that two dot products may be more than the f32 range apart and their
 // scores still close takes the products by c first (M c is then below 2^9); one
 // whose c would pass the range keeps the scale, where any two scores that
@@ -1821,7 +1823,7 @@ __device__ __forceinline__ RowExp causal_exp(const PrefillArgs &a, float m, bool
     // kernel of 32 tiles at D = 128 runs one wave per SIMD instead of two
     const float c = __uint_as_float(
         __builtin_amdgcn_readfirstlane(__float_as_uint(s >= 0x1p127f ? s : s * 1.442695f)));
-    RowExp x{m, c, over ? __builtin_fmaf(sm - a.sink, 1.442695f, 0.5f) : 0.5f};
+    RowExp x{m, c, __builtin_fmaf(over ? sm - a.sink : 0.0f * sm, 1.442695f, 0.5f)};
     if (s < 0x1p-120f) {
         x.X = 0.0f;
         x.b -= m * x.c;

@@ -15,7 +15,7 @@ import torch
 import hsdpa
 import oracle
 from hsdpa import workloads as W
-from parity import assert_parity
+from parity import assert_parity, bf16_f32
 
 pytestmark = pytest.mark.gpu
 
@@ -89,6 +89,26 @@ def test_tiny_scale(torch_cuda, case):
     w = _workload(f"{name}_tiny", h, kvh, d, rows, past, 104, 2.0 ** -126, signs=True)
     _, out = _run(w)
     assert_parity(out, oracle.attention(w), w, w.name)
+
+
+@pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
+def test_overflowing_scores(torch_cuda, case):
+    """Scores past the f32 range: the largest is infinite, its difference from
+    itself a NaN, which the exponential clamps like the others' -inf, so that every
+    key weighs the same, 2^-126. Those weights' products are at the edge of what
+    the matrix cores keep (smaller ones are flushed, an error of 1 a key at most before
+    the division by the number of keys), so the outputs are not compared one by one: over
+    32 keys or more the mean of N(0,1) values lies below 1 (6 of its deviations), the
+    flushed products add 1 at most, and a single key's values, as one infinite score would give
+    them, pass 2 in a row of 64 values or more almost surely."""
+    name, h, kvh, d, rows, past, sink, _ = case
+    w = W.make(name, heads=h, kv_heads=kvh, head_dim=d, rows=rows, past=past, seed=34, scale=3e38)
+    s = 3.0 if sink else None
+    _, out = _run(w, s)
+    assert np.isfinite(bf16_f32(out)).all()
+    for x in (out, oracle.attention(w, sink=s)):
+        x = np.abs(bf16_f32(x).reshape(rows, h, d))[max(0, 31 - past):]
+        assert x.max() <= 2.0
 
 
 @pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
