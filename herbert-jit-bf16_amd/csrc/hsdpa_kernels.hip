@@ -414,7 +414,7 @@ bool prefill_flat_shape(const PrefillArgs &a, int head_dim, int heads, const Pre
     // launches take more or less than the equal shares' (prefill_flat), and with
     // the sink that its kernels stage K and V for each head: fitted to 650 calls
     // timed both ways and shifted so that neither side loses much, on 300 other
-    // calls at most 6 % against the better one
+    // calls at most 8 % against the better one
     const uint64_t other =
         splits > 1 ? 4 * ((tiles + splits - 1) / splits) + (a.sink_on ? 20 : 9)
         : pr.srows ? 17 * pr.longest / 5 + 12 * a.rows * static_cast<uint64_t>(heads) / 10000 + 4
